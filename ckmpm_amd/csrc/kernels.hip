@@ -34,6 +34,10 @@ constexpr uint32_t kRebinScanTile = kThreads * kRebinScanItems;
 static_assert(kRebinScanTile % kCountTile == 0, "scan tiles hold whole count tiles");
 
 __device__ __forceinline__ uint32_t LaneId() { return __lane_id(); }
+// A wave-uniform value, kept in a scalar register.
+__device__ __forceinline__ float Uniform(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
 
 __device__ __forceinline__ uint32_t WaveInclusiveScan(uint32_t v) {
     const uint32_t lane = LaneId();
@@ -61,6 +65,15 @@ __device__ __forceinline__ uint32_t BlockExclusiveScan(uint32_t v, uint32_t& tot
     __syncthreads();
     total = tot;
     return wbase + inc - v;
+}
+
+// Element i < 2^29 of a wave-uniform array: a scalar base and a 32-bit byte offset, so a
+// particle's loads and stores share one vector offset (no 64-bit address per attribute).
+__device__ __forceinline__ float Ld(const float* base, uint32_t i) {
+    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + (i << 2));
+}
+__device__ __forceinline__ void St(float* base, uint32_t i, float v) {
+    *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + (i << 2)) = v;
 }
 
 // Number of set bits of a wave mask below this lane (mbcnt).
@@ -821,25 +834,38 @@ __global__ __launch_bounds__(kThreads) void GridUpdateKernel(GridUpdateArgs a) {
 // node is flushed once with a global float atomic.  The kernel also emits each
 // particle's block move (direction) and its deterministic rank among the block's
 // particles with the same move, for the counting-sort rebin.
-constexpr int kWin = 512;  // 8^3 nodes of one sub-grid window
-
 // LDS windows of a particle block (node coordinates relative to the block's first
-// node, 0..7 over the block and its +1 neighbours).  Stencil bases lie in [1,6] for
-// grid 0 and [0,6] for grid 1 (window check), so grid 0 uses nodes [1,7]^3 and grid 1
-// nodes [0,7]^3: 343 + 512 nodes per channel instead of 2 x 512.
-constexpr int kM0Win = 343;              // 7^3
-constexpr int kMWin = kM0Win + 512;      // both sub-grids, one channel
-// Halo entry (block o of the 2x2x2 neighbourhood b + {0,1}^3, bit 2 = x, bit 1 = y,
-// bit 0 = z; node nd = g*64 + x*16 + y*4 + z of its 128) -> window entry, or -1 for a
-// grid-0 node outside [1,7]^3.  The halo load and the flush walk the neighbourhood block
-// by block, so a wavefront reads or updates 64 consecutive nodes of one grid block.
-__device__ __forceinline__ int WindowOfHalo(int o, int nd) {
-    const int lx = ((o >> 2) & 1) * 4 + ((nd >> 4) & 3);
-    const int ly = ((o >> 1) & 1) * 4 + ((nd >> 2) & 3);
-    const int lz = (o & 1) * 4 + (nd & 3);
-    if (nd >= 64) return kM0Win + lx * 64 + ly * 8 + lz;
+// node, 0..7 over the block and its +1 neighbours).
+//   P2G accumulator: the particles' new stencil bases lie in [1,6] for grid 0 and [0,6]
+//     for grid 1 (window check), so nodes [1,7]^3 and [0,7]^3.
+//   velocity: the old bases lie in the block's cells 2..5 (grid 0) and 1..5 (grid 1), so
+//     nodes [2,6]^3 and [1,6]^3: 341 of the 855 entries of the accumulator's windows.
+// Strides (in entries) of y and x.  A chunk's lanes cycle through the block's 4^3 cells,
+// z fastest, so lanes 16 apart differ by the x stride and lanes 4 apart by the y stride.
+// The 8-byte accumulator deposits of 32 such lanes fall on 32 distinct LDS bank pairs
+// when x = 4 and y = 8 modulo 32; with the dense strides (7, 49 and 8, 64) two to four of
+// them share a pair.  Padding took the bank-conflict cycles of the 5M-particle fluid
+// launch from 62M to 46M, its substep from 24.8 to 24.0 ms per 40 and the 1M jelly's from
+// 6.28 to 5.77.  Padding the 4-byte velocity windows the same way gave nothing.
+constexpr int kM0Y = 8, kM0X = 60, kM1Y = 8, kM1X = 68;
+constexpr int kV0Y = 5, kV0X = 25, kV1Y = 6, kV1X = 36;
+constexpr int kM0Win = 6 * kM0X + 6 * kM0Y + 7;
+constexpr int kMWin = kM0Win + 7 * kM1X + 7 * kM1Y + 8;  // both sub-grids, one channel
+constexpr int kV0Win = 4 * kV0X + 4 * kV0Y + 5;
+constexpr int kVWin = kV0Win + 5 * kV1X + 5 * kV1Y + 6;
+constexpr int kCoreNodes = 125 + 216;    // nodes in reach of the block's own cells 2..5
+constexpr int kCoreColumns = 2 * (25 + 36);  // their z columns, one per block and (x, y)
+// Accumulator entry of node (x, y, z) of sub-grid g, or -1 for a grid-0 node outside [1,7]^3.
+__device__ __forceinline__ int MEntry(int g, int lx, int ly, int lz) {
+    if (g) return kM0Win + lx * kM1X + ly * kM1Y + lz;
     if (lx == 0 || ly == 0 || lz == 0) return -1;
-    return (lx - 1) * 49 + (ly - 1) * 7 + (lz - 1);
+    return (lx - 1) * kM0X + (ly - 1) * kM0Y + (lz - 1);
+}
+// Accumulator entry of node nd = g*64 + x*16 + y*4 + z of block o of the 2x2x2
+// neighbourhood b + {0,1}^3 (bit 2 = x, bit 1 = y, bit 0 = z), or -1.
+__device__ __forceinline__ int WindowOfHalo(int o, int nd) {
+    return MEntry(nd >> 6, ((o >> 2) & 1) * 4 + ((nd >> 4) & 3), ((o >> 1) & 1) * 4 + ((nd >> 2) & 3),
+                  (o & 1) * 4 + (nd & 3));
 }
 
 // P2G accumulator in LDS: 64-bit fixed point.  On gfx950 a wavefront's ds_add_f32
@@ -898,8 +924,7 @@ __device__ __forceinline__ void DepositP2G(LdsAcc* sM, const Stencil32 (&sn)[2],
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
         const Stencil32& sg = sn[g];
-        // grid 0: nodes [1,7]^3 (7 wide), grid 1: nodes [0,7]^3 (8 wide)
-        const int s1 = g ? 8 : 7, s2 = g ? 64 : 49, lo = g ? 0 : 1;
+        const int s1 = g ? kM1Y : kM0Y, s2 = g ? kM1X : kM0X, lo = g ? 0 : 1;
         LdsAcc* base = sM + (g ? kM0Win : 0) + (sg.c[0] - lo) * s2 + (sg.c[1] - lo) * s1 + (sg.c[2] - lo);
         float pa[3];
         double pad[3];
@@ -947,6 +972,30 @@ __device__ __forceinline__ void DepositP2G(LdsAcc* sM, const Stencil32 (&sn)[2],
     }
 }
 
+// G2P of one sub-grid from the halo blocks in global memory, for a stencil outside the
+// velocity window: adds to v (sum of both grids) and B (in units of dx).
+__device__ __forceinline__ void GatherG2P(int g, const Stencil32& s, const uint32_t* sHalo, const float* V, float (&v)[3],
+                                          float (&B)[9]) {
+#pragma unroll 1
+    for (int o = 0; o < 8; ++o) {
+        const int ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
+        const int lx = min(max(s.c[0] + ox, 0), 7), ly = min(max(s.c[1] + oy, 0), 7), lz = min(max(s.c[2] + oz, 0), 7);
+        const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2)];
+        if (bi == kEmpty) continue;
+        const float* src = V + static_cast<size_t>(bi) * kVFloats + g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3);
+        const float w = NodeWeight(s, ox, oy, oz);
+        const float d[3] = {static_cast<float>(ox) - s.t[0], static_cast<float>(oy) - s.t[1],
+                            static_cast<float>(oz) - s.t[2]};
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const float wv = w * src[128 * r];
+            v[r] += wv;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) B[r * 3 + c] = fmaf(wv, d[c], B[r * 3 + c]);
+        }
+    }
+}
+
 // Particles are taken in 64-particle chunks, one wavefront per chunk (chunk c of a block
 // goes to wave c mod waves): with a few hundred particles per block, 256-particle
 // chunks would leave about a quarter of the lanes idle.  The rank of a particle among
@@ -958,12 +1007,12 @@ constexpr int kRoundChunks = 12;
 constexpr uint32_t kRoundParticles = kRoundChunks * 64;
 constexpr int kHistStride = 28;  // per chunk: 27 move counts (then prefixes), padded
 
-// 4 waves per SIMD: LDS (40.1 KiB per workgroup) allows 4 workgroups per CU; this caps
+// 4 waves per SIMD: LDS (37.2 KiB per workgroup) allows 4 workgroups per CU; this caps
 // the VGPRs at 128
 template <int KIND, int THREADS>
 __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint32_t ng) {
     constexpr uint32_t kWaves = THREADS / 64;
-    __shared__ float sV[kVChannels * kMWin];
+    __shared__ float sV[kVChannels * kVWin];
     __shared__ __align__(16) LdsAcc sM[kMChannels * kMWin];
     __shared__ uint16_t sCode[kRoundParticles];               // move | rank in the chunk << 5
     __shared__ uint16_t sHist[kRoundChunks * kHistStride];    // per chunk and move
@@ -971,6 +1020,7 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
     __shared__ uint32_t sRun[32];   // particles of the block per move before this round
     __shared__ uint32_t sTot[32];   // particles per move in this round
     __shared__ uint32_t sBlkMax;    // largest deposit bound of the block (FP32 bits)
+    __shared__ uint32_t sMoved;     // a particle of the block has left its cells
     __shared__ uint32_t sGlobal;    // particles of the block deposited with global atomics
 
     const uint32_t A = a.lc->A, Nb = a.lc->Nb;
@@ -987,7 +1037,6 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
         if (!(ref <= 1.0e37f)) ref = 1.0e37f;  // a non-finite grid is already flagged
         if (ref > 0.0f) mexp = max(kMinExp, static_cast<int>((__float_as_uint(ref) >> 23) & 0xFFu) - 127 + 2);
     }
-    const float fast_limit = __int_as_float((mexp - 1 + 127) << 23);  // 2^(mexp-1)
 
     // The accumulator and the move counts are cleared once here; the flush and the
     // prefix pass leave them zero for the next block.  16-byte clears (the size is even).
@@ -1006,9 +1055,9 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
             if (tid == 0) a.blkmax[j] = 0.0f;
             continue;
         }
-        int bb[3];
-        CoordsOf(a.dom, a.keys[j], bb[0], bb[1], bb[2]);
         if (tid < 8) {
+            int bb[3];
+            CoordsOf(a.dom, a.keys[j], bb[0], bb[1], bb[2]);
             const int bx = bb[0] + ((tid >> 2) & 1), by = bb[1] + ((tid >> 1) & 1), bz = bb[2] + (tid & 1);
             uint32_t bi = kEmpty;
             if (InDomain(a.dom, bx, by, bz)) bi = a.table[KeyOf(a.dom, bx, by, bz)];
@@ -1019,6 +1068,7 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
         if (tid == 0) {
             sBlkMax = 0u;
             sGlobal = 0u;
+            sMoved = 0u;
         }
         // fixed-point scales of this block (LdsAcc): weights 2^kq, momentum 2^(kq - mexp)
         const uint32_t nblk = end - beg;
@@ -1028,28 +1078,34 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
         const double wscale = __longlong_as_double(static_cast<long long>(kq + 1023) << 52);  // 2^kq
         const float qs = __int_as_float((kq - mexp + 127) << 23);                             // 2^(kq - mexp)
         const float inv_qs = __int_as_float((mexp - kq + 127) << 23);
-        float tmax = 0.0f;  // largest deposit bound of this thread's particles
+        const float fast_limit_q = __int_as_float((kq - 1 + 127) << 23);  // 2^(mexp-1) scaled by qs
+        // uniform factors of the particle loop, in scalar registers; the momentum factors
+        // carry the fixed-point scale qs (a power of two)
+        const float half_dt = Uniform(0.5f * a.dt);
+        const float mass_q = Uniform(0.5f * a.mat.mass * qs);
+        const float mdx_q = Uniform(a.mat.mass * dx * qs);
+        const float stress_q = Uniform(2.0f * a.next_dt * a.mat.volume * inv_dx * qs);
+        float tmax = 0.0f;  // largest deposit bound of this thread's particles, scaled by qs
         __syncthreads();
-        // velocity halo in the same windows as the P2G accumulator (3 channels): a thread
-        // takes a z column of 4 nodes of a grid block (16-byte loads), which fills 4
-        // consecutive window entries; in grid 0 the first of them lies outside the window
-        // when the block is at z offset 0 (lz = 0), and a column at lx = 0 or ly = 0
-        // lies outside altogether
-        for (int e = tid; e < 8 * kNodesPerBlock / 4; e += THREADS) {
-            const int o = e >> 5, nd0 = (e & 31) * 4;
-            const int r3 = WindowOfHalo(o, nd0 + 3);
-            if (r3 < 0) continue;
-            const uint32_t bi = sHalo[o];
-            const float4* src = reinterpret_cast<const float4*>(a.V + static_cast<size_t>(bi) * kVFloats + nd0);
-            const bool first = nd0 >= 64 || (o & 1);
+        // velocity halo: a thread takes a z column of 4 nodes of a grid block (16-byte loads)
+        // and stores the nodes inside the window: z = lo..3 of the block at z offset 0, 4..6
+        // of the one above
+        for (int e = tid; e < kCoreColumns; e += THREADS) {
+            const bool g1 = e < 72;
+            const int col = (g1 ? e : e - 72) >> 1, zb = e & 1, lo = g1 ? 1 : 2;
+            const int lx = (g1 ? col / 6 : col / 5) + lo, ly = col - (lx - lo) * (g1 ? 6 : 5) + lo;
+            const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | zb];
+            const float4* src = reinterpret_cast<const float4*>(a.V + static_cast<size_t>(bi) * kVFloats + (g1 ? 64 : 0) +
+                                                                (lx & 3) * 16 + (ly & 3) * 4);
+            const int r0 = (g1 ? kV0Win + (lx - 1) * kV1X + (ly - 1) * kV1Y : (lx - 2) * kV0X + (ly - 2) * kV0Y) +
+                           (zb ? 4 - lo : 0);
 #pragma unroll
             for (int ch = 0; ch < kVChannels; ++ch) {
                 const float4 v = bi != kEmpty ? src[32 * ch] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                const int r = ch * kMWin + r3;
-                if (first) sV[r - 3] = v.x;
-                sV[r - 2] = v.y;
-                sV[r - 1] = v.z;
-                sV[r] = v.w;
+                float* d = sV + ch * kVWin + r0;
+                d[0] = zb ? v.x : (g1 ? v.y : v.z);
+                d[1] = zb ? v.y : (g1 ? v.z : v.w);
+                if (zb || g1) d[2] = zb ? v.z : v.w;
             }
         }
         if (tid == 0) {
@@ -1073,6 +1129,7 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
                 const uint32_t pe = pe_next;
                 if (c + kWaves < nch && (c + kWaves) * 64u + lane < rn) pe_next = a.perm[t + kWaves * 64u];
                 uint32_t dir = 31u;
+                bool stays = true;
                 if (active) {
                     uint32_t s = pe & kSlotMask;
                     int mv = static_cast<int>(pe >> kMoveShift);
@@ -1088,64 +1145,49 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
                     float x[3], F[9], q = 0.0f, logJp = 0.0f;  // F holds E = F - I; q = J - 1 (fluid)
 #pragma unroll
                     for (int k = 0; k < 3; ++k)
-                        x[k] = __fsub_rn(a.st_in[k * N + s], __fmul_rn(static_cast<float>(4 * mov[k]), dx));
+                        x[k] = __fsub_rn(Ld(a.st_in + k * N, s), __fmul_rn(static_cast<float>(4 * mov[k]), dx));
                     if (KIND == kFluid) {
-                        q = a.st_in[3 * N + s];
+                        q = Ld(a.st_in + 3 * N, s);
                     } else {
 #pragma unroll
-                        for (int k = 0; k < 9; ++k) F[k] = a.st_in[(3 + k) * N + s];
-                        if (KIND == kDruckerPrager || KIND == kCamClay) logJp = a.st_in[12 * N + s];
+                        for (int k = 0; k < 9; ++k) F[k] = Ld(a.st_in + (3 + k) * N, s);
+                        if (KIND == kDruckerPrager || KIND == kCamClay) logJp = Ld(a.st_in + 12 * N, s);
                     }
                     float lam = a.mat.lambda, mu = a.mat.mu;
                     if (a.pp_attr) {
-                        lam = a.st_in[a.pp_attr * N + s];
-                        mu = a.st_in[(a.pp_attr + 1) * N + s];
+                        lam = Ld(a.st_in + a.pp_attr * N, s);
+                        mu = Ld(a.st_in + (a.pp_attr + 1) * N, s);
                     }
-                    const float rigid = a.rigid_attr ? a.st_in[a.rigid_attr * N + s] : 0.0f;
+                    const float rigid = a.rigid_attr ? Ld(a.st_in + a.rigid_attr * N, s) : 0.0f;
                     // ---------------- G2P at x (both sub-grids, 16 nodes)
                     float xs[3];
 #pragma unroll
                     for (int k = 0; k < 3; ++k) xs[k] = __fmul_rn(x[k], inv_dx);
-                    float v[3] = {0.f, 0.f, 0.f}, B[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                    float D[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                    bool bad = false;
+                    // v: sum of both grids (twice the velocity); B in units of dx
+                    float v[3], B[9], Di[6], C[9];
                     Stencil32 sp[2];
-                    MakeStencilPair(xs, sp[0], sp[1]);
+                    {
+                        // The binned cell (2..5 in the frame of the block that binned the
+                        // particle) can move by one in this block's frame through FP32 rounding
+                        // of + 0.25; the stencil keeps the base cells 2..5.
+                        float sn[3], diag[3];
+                        MakeStencilPair<2, 5>(xs, sp[0], sp[1], sn, diag);
+                        MomentInverse(sn, diag, inv_dx, Di);
+                    }
 #pragma unroll
                     for (int g = 0; g < 2; ++g) {
                         const Stencil32& sg = sp[g];
-                        int l[3];
-                        float m1[3];
-#pragma unroll
-                        for (int k = 0; k < 3; ++k) {
-                            const int lc = sg.c[k];
-                            // the binned cell (2..5 in the frame of the block that binned the
-                            // particle) can move by one in this block's frame through FP32
-                            // rounding of + 0.25, so the bases lie in [1,6] (grid 0), [0,6] (grid 1)
-                            const int lo = g ? 0 : 1;
-                            bad |= lc < lo || lc > 6;
-                            l[k] = min(max(lc, lo), 6) - lo;
-                            // D closed form per axis: second moment on the diagonal, products of
-                            // first moments off the diagonal (units of dx^2)
-                            const float w0 = sg.w0[k], w1 = 1.0f - w0, tt = sg.t[k];
-                            m1[k] = w1 - tt;
-                            D[k * 4] += w0 * tt * tt + w1 * (1.0f - tt) * (1.0f - tt);
-                        }
-                        D[1] += m1[0] * m1[1];
-                        D[2] += m1[0] * m1[2];
-                        D[5] += m1[1] * m1[2];
+                        const int s1 = g ? kV1Y : kV0Y, s2 = g ? kV1X : kV0X, lo = g ? 1 : 2;
+                        const float* base = sV + (g ? kV0Win : 0) + (sg.c[0] - lo) * s2 + (sg.c[1] - lo) * s1 + (sg.c[2] - lo);
                         // B = sum_i v_i (x_i - x_p)^T w_i with x_i - x_p = (o - t) dx per axis:
                         // B_rc = dx (S_rc - vg_r t_c), S_rc = sum over the nodes with o_c = 1 of w v_r.
                         // The weights are a tensor product, so vg and S are contracted axis by
                         // axis (z, then y, then x): 22 instructions per channel.
-                        const int s1 = g ? 8 : 7, s2 = g ? 64 : 49;
-                        const float* base = sV + (g ? kM0Win : 0) + l[0] * s2 + l[1] * s1 + l[2];
                         const float wx0 = sg.w0[0], wy0 = sg.w0[1], wz0 = sg.w0[2];
                         const float wx1 = 1.0f - wx0, wy1 = 1.0f - wy0, wz1 = 1.0f - wz0;
-                        float vg[3], S[9];
 #pragma unroll
                         for (int r = 0; r < 3; ++r) {
-                            const float* vr = base + r * kMWin;
+                            const float* vr = base + r * kVWin;
                             float T[4], U[4];  // per (x, y) column: sum over z, z-moment
 #pragma unroll
                             for (int q = 0; q < 4; ++q) {
@@ -1160,34 +1202,36 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
                                 P[ox] = fmaf(wy0, T[ox * 2], Q[ox]);
                                 Z[ox] = fmaf(wy0, U[ox * 2], wy1 * U[ox * 2 + 1]);
                             }
-                            S[r * 3 + 0] = wx1 * P[1];
-                            vg[r] = fmaf(wx0, P[0], S[r * 3 + 0]);
-                            S[r * 3 + 1] = fmaf(wx0, Q[0], wx1 * Q[1]);
-                            S[r * 3 + 2] = fmaf(wx0, Z[0], wx1 * Z[1]);
-                        }
+                            const float S0 = wx1 * P[1];
+                            const float vg = fmaf(wx0, P[0], S0);
+                            const float S[3] = {S0, fmaf(wx0, Q[0], wx1 * Q[1]), fmaf(wx0, Z[0], wx1 * Z[1])};
+                            v[r] = g ? v[r] + vg : vg;
 #pragma unroll
-                        for (int r = 0; r < 3; ++r) {
-                            v[r] += vg[r];
-#pragma unroll
-                            for (int c = 0; c < 3; ++c) B[r * 3 + c] += dx * (S[r * 3 + c] - vg[r] * sg.t[c]);
+                            for (int c = 0; c < 3; ++c) {
+                                const float b = fmaf(-vg, sg.t[c], S[c]);
+                                B[r * 3 + c] = g ? B[r * 3 + c] + b : b;
+                            }
                         }
                     }
-                    if (bad) SetFlag(a.st, kFlagOutOfWindow);
-                    const float dx2 = dx * dx;
-                    D[0] *= dx2;
-                    D[4] *= dx2;
-                    D[8] *= dx2;
-                    D[1] *= dx2;
-                    D[2] *= dx2;
-                    D[5] *= dx2;
-                    D[3] = D[1];
-                    D[6] = D[2];
-                    D[7] = D[5];
-                    float Di[9], C[9];
-                    InverseSym3(D, Di);
-                    MatMul3(B, Di, C);
+                    // A position farther out (an imported state) takes its own stencil from the
+                    // grid blocks themselves; base cells beyond 1..6 are an error.
+                    float out = 0.0f;
 #pragma unroll
-                    for (int k = 0; k < 3; ++k) v[k] *= 0.5f;
+                    for (int k = 0; k < 3; ++k) out = fmaxf(out, fabsf(sp[0].t[k] - 0.5f));
+                    if (!(out <= 0.5001f)) {
+                        float sn[3], diag[3];
+                        MakeStencilPair(xs, sp[0], sp[1], sn, diag);
+                        MomentInverse(sn, diag, inv_dx, Di);
+                        uint32_t far = 0u;
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) far = max(far, static_cast<uint32_t>(sp[0].c[k] - 1));
+                        if (far > 5u) SetFlag(a.st, kFlagOutOfWindow);
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) v[k] = B[3 * k] = B[3 * k + 1] = B[3 * k + 2] = 0.0f;
+                        GatherG2P(0, sp[0], sHalo, a.V, v, B);
+                        GatherG2P(1, sp[1], sHalo, a.V, v, B);
+                    }
+                    MatMulSym3(B, Di, C);  // C = B D^-1
                     if (rigid != 0.0f) {
                         // a rigid particle takes nothing from the grid and moves at the
                         // prescribed velocity (mpm_algorithm.cuh:1609-1617)
@@ -1200,7 +1244,7 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
                         }
                     } else {
 #pragma unroll
-                        for (int k = 0; k < 3; ++k) x[k] += a.dt * v[k];
+                        for (int k = 0; k < 3; ++k) x[k] = fmaf(half_dt, v[k], x[k]);
                     }
                     // ---------------- deformation update and stress
                     float tau[9];
@@ -1219,85 +1263,68 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
                         else StressCamClay(a.mat, lam, mu, F, logJp, tau);
                     }
 #pragma unroll
-                    for (int k = 0; k < 3; ++k) a.st_out[k * N + t] = x[k];
+                    for (int k = 0; k < 3; ++k) St(a.st_out + k * N, t, x[k]);
                     if (KIND == kFluid) {
-                        a.st_out[3 * N + t] = q;
+                        St(a.st_out + 3 * N, t, q);
                     } else {
 #pragma unroll
-                        for (int k = 0; k < 9; ++k) a.st_out[(3 + k) * N + t] = F[k];
-                        if (KIND == kDruckerPrager || KIND == kCamClay) a.st_out[12 * N + t] = logJp;
+                        for (int k = 0; k < 9; ++k) St(a.st_out + (3 + k) * N, t, F[k]);
+                        if (KIND == kDruckerPrager || KIND == kCamClay) St(a.st_out + 12 * N, t, logJp);
                     }
                     if (a.pp_attr) {
-                        a.st_out[a.pp_attr * N + t] = lam;
-                        a.st_out[(a.pp_attr + 1) * N + t] = mu;
+                        St(a.st_out + a.pp_attr * N, t, lam);
+                        St(a.st_out + (a.pp_attr + 1) * N, t, mu);
                     }
-                    if (a.rigid_attr) a.st_out[a.rigid_attr * N + t] = rigid;
-                    // ---------------- block move for the rebin (FP32 grid-0 binning)
-                    int dlt[3];
-                    bool clamped = false;
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        const int dd = FloorDiv4(Cell0(x[k], inv_dx) - 2);
-                        clamped |= dd < -1 || dd > 1;
-                        dlt[k] = min(max(dd, -1), 1);
-                    }
-                    if (clamped) SetFlag(a.st, kFlagOutOfWindow);
-                    if (!InDomain(a.dom, bb[0] + dlt[0], bb[1] + dlt[1], bb[2] + dlt[2])) {
-                        SetFlag(a.st, kFlagOutOfDomain);
-                        dlt[0] = dlt[1] = dlt[2] = 0;
-                    }
-                    dir = static_cast<uint32_t>((dlt[0] + 1) * 9 + (dlt[1] + 1) * 3 + (dlt[2] + 1));
+                    if (a.rigid_attr) St(a.st_out + a.rigid_attr * N, t, rigid);
                     // ---------------- P2G at the new x
 #pragma unroll
                     for (int k = 0; k < 3; ++k) xs[k] = __fmul_rn(x[k], inv_dx);
                     Stencil32 sn[2];
-                    MakeStencilPair(xs, sn[0], sn[1]);
-                    bool inwin = true;
-                    float Dn[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                    float Dh[6];
+                    {
+                        float s3[3], diag[3];
+                        MakeStencilPair(xs, sn[0], sn[1], s3, diag);
+                        MomentInverse(s3, diag, stress_q, Dh);
+                    }
+                    // ---------------- block move for the rebin: the grid-0 base cell is the FP32
+                    // binning cell, 2..5 in the block's frame while the particle stays
+                    uint32_t far = 0u;
 #pragma unroll
-                    for (int g = 0; g < 2; ++g) {
-                        float m1[3];
+                    for (int k = 0; k < 3; ++k) far = max(far, static_cast<uint32_t>(sn[0].c[k] - 2));
+                    dir = 13u;
+                    stays = far <= 3u;
+                    if (!stays) {
+                        int dlt[3];
+                        bool clamped = false;
 #pragma unroll
                         for (int k = 0; k < 3; ++k) {
-                            const int lc = sn[g].c[k];
-                            inwin &= g == 0 ? (lc >= 1 && lc <= 6) : (lc >= 0 && lc <= 6);
-                            const float w0 = sn[g].w0[k], w1 = 1.0f - w0, tt = sn[g].t[k];
-                            m1[k] = w1 - tt;
-                            Dn[k * 4] += w0 * tt * tt + w1 * (1.0f - tt) * (1.0f - tt);
+                            const int dd = FloorDiv4(sn[0].c[k] - 2);
+                            clamped |= dd < -1 || dd > 1;
+                            dlt[k] = min(max(dd, -1), 1);
                         }
-                        Dn[1] += m1[0] * m1[1];
-                        Dn[2] += m1[0] * m1[2];
-                        Dn[5] += m1[1] * m1[2];
+                        if (clamped) SetFlag(a.st, kFlagOutOfWindow);
+                        int bb[3];
+                        CoordsOf(a.dom, a.keys[j], bb[0], bb[1], bb[2]);
+                        if (!InDomain(a.dom, bb[0] + dlt[0], bb[1] + dlt[1], bb[2] + dlt[2])) {
+                            SetFlag(a.st, kFlagOutOfDomain);
+                            dlt[0] = dlt[1] = dlt[2] = 0;
+                        }
+                        dir = static_cast<uint32_t>((dlt[0] + 1) * 9 + (dlt[1] + 1) * 3 + (dlt[2] + 1));
                     }
-                    if (!inwin) {
+                    uint32_t wide = 0u;  // stencil bases outside the window ([1,6] of grid 0)
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) wide = max(wide, static_cast<uint32_t>(sn[0].c[k] - 1));
+                    if (wide > 5u) {
                         SetFlag(a.st, kFlagOutOfWindow);
                     } else {
-                        // D^ = (0.5 D')^-1 = 2 D'^-1; K = m C - nextDt V D^ tau
-                        const float h = 0.5f * dx2;
-                        Dn[0] *= h;
-                        Dn[4] *= h;
-                        Dn[8] *= h;
-                        Dn[1] *= h;
-                        Dn[2] *= h;
-                        Dn[5] *= h;
-                        Dn[3] = Dn[1];
-                        Dn[6] = Dn[2];
-                        Dn[7] = Dn[5];
-                        float Dh[9], DT[9], K[9];
-                        InverseSym3(Dn, Dh);
-                        MatMul3(Dh, tau, DT);
-                        const float sv = a.next_dt * a.mat.volume;
+                        // D^ = (0.5 D')^-1 = 2 D'^-1; K = m C - nextDt V D^ tau.  Node momentum
+                        // m v + K (x_i - x_p), x_i - x_p = (o - t) dx: = a + sum_c o_c kc_c with
+                        // a = m v - dx K t and kc_c = dx K e_c; all in the fixed-point scale qs,
+                        // which the uniform factors hold (stress_q is in Dh)
+                        float pm[3], kc[3][3];
 #pragma unroll
-                        for (int k = 0; k < 9; ++k) K[k] = C[k] * a.mat.mass - sv * DT[k];
-                        float pm[3], kc[3][3];  // m v and dx K e_c
-#pragma unroll
-                        for (int r = 0; r < 3; ++r) pm[r] = a.mat.mass * v[r];
-                        // node momentum m v + K (x_i - x_p), x_i - x_p = (o - t) dx:
-                        // = a + sum_c o_c kc_c with a = m v - dx K t and kc_c = dx K e_c
-#pragma unroll
-                        for (int c = 0; c < 3; ++c)
-#pragma unroll
-                            for (int r = 0; r < 3; ++r) kc[c][r] = dx * K[r * 3 + c];
+                        for (int r = 0; r < 3; ++r) pm[r] = mass_q * v[r];
+                        SymMulSub(Dh, tau, mdx_q, C, kc);
                         float bound = 0.0f, bsum = fabsf(x[0]) + fabsf(x[1]) + fabsf(x[2]);
 #pragma unroll
                         for (int r = 0; r < 3; ++r) {
@@ -1311,13 +1338,7 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
                             SetFlag(a.st, kFlagNonFinite);
                         } else {
                             tmax = fmaxf(tmax, bound);
-#pragma unroll
-                            for (int r = 0; r < 3; ++r) {
-                                pm[r] *= qs;
-#pragma unroll
-                                for (int c = 0; c < 3; ++c) kc[c][r] *= qs;
-                            }
-                            if (bound < fast_limit) {
+                            if (bound < fast_limit_q) {
                                 DepositP2G<false>(sM, sn, pm, kc, wscale, inv_qs, sHalo, a.M);
                             } else {
                                 DepositP2G<true>(sM, sn, pm, kc, wscale, inv_qs, sHalo, a.M);
@@ -1328,45 +1349,56 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
                         }
                     }
                 }
-                // ---------------- rank among the chunk's particles with the same move
-                const uint64_t peers = MatchPeers<5>(dir);
-                const uint32_t rank = LanesBelow(peers);
-                if (active) {
-                    sCode[t - r0] = static_cast<uint16_t>(dir | (rank << 5));
-                    if (rank == 0) sHist[c * kHistStride + dir] = static_cast<uint16_t>(__popcll(peers));
+                // ---------------- rank among the chunk's particles with the same move (all of
+                // them stay in most chunks: the rank is then the lane)
+                if (__all(stays)) {
+                    if (active) sCode[t - r0] = static_cast<uint16_t>(13u | (lane << 5));
+                    if (lane == 0) sHist[c * kHistStride + 13] = static_cast<uint16_t>(min(64u, rn - c * 64u));
+                } else {
+                    const uint64_t peers = MatchPeers<5>(dir);
+                    const uint32_t rank = LanesBelow(peers);
+                    if (active) {
+                        sCode[t - r0] = static_cast<uint16_t>(dir | (rank << 5));
+                        if (rank == 0) sHist[c * kHistStride + dir] = static_cast<uint16_t>(__popcll(peers));
+                    }
+                    if (lane == 0) sMoved = 1u;
                 }
             }
             // largest deposit bound of the block (for the next substep's scale): one LDS
             // max per wave instruction (non-negative floats order as their bits)
-            if (last && tmax > 0.0f) atomicMax(&sBlkMax, __float_as_uint(tmax));
+            if (last && tmax > 0.0f) atomicMax(&sBlkMax, __float_as_uint(tmax * inv_qs));
             __syncthreads();
-            // exclusive prefix of each move's counts over the round's chunks
-            if (tid < kDirections) {
-                uint32_t run = 0;
-                for (uint32_t c = 0; c < nch; ++c) {
-                    const uint32_t h = sHist[c * kHistStride + tid];
-                    sHist[c * kHistStride + tid] = static_cast<uint16_t>(run);
-                    run += h;
+            // While no particle of the block has moved, a particle's rank is its position in
+            // the block; otherwise an exclusive prefix of each move's counts over the
+            // round's chunks gives it.
+            const bool moved = sMoved != 0u;
+            if (moved) {
+                if (tid < kDirections) {
+                    uint32_t run = 0;
+                    for (uint32_t c = 0; c < nch; ++c) {
+                        const uint32_t h = sHist[c * kHistStride + tid];
+                        sHist[c * kHistStride + tid] = static_cast<uint16_t>(run);
+                        run += h;
+                    }
+                    sTot[tid] = run;
                 }
-                sTot[tid] = run;
-            }
-            __syncthreads();
-            for (uint32_t i = tid; i < rn; i += THREADS) {
-                const uint32_t v = sCode[i], dir = v & 31u;
-                const uint32_t r = sRun[dir] + sHist[(i >> 6) * kHistStride + dir] + (v >> 5);
-                a.code[r0 + i] = dir | (r << 5);
+                __syncthreads();
+                for (uint32_t i = tid; i < rn; i += THREADS) {
+                    const uint32_t v = sCode[i], dir = v & 31u;
+                    const uint32_t r = sRun[dir] + sHist[(i >> 6) * kHistStride + dir] + (v >> 5);
+                    a.code[r0 + i] = dir | (r << 5);
+                }
+            } else {
+                for (uint32_t i = tid; i < rn; i += THREADS) a.code[r0 + i] = 13u | ((r0 - beg + i) << 5);
             }
             if (last) {
-                // ---------------- flush: one global atomic per non-zero node and channel,
-                // block by block of the neighbourhood (fixed point -> FP32 through an exact
-                // double, 2^-kq m for the weights, 2^(mexp-kq) for the momentum); every entry
-                // read non-zero is cleared for the next block
+                // ---------------- flush: one global atomic per non-zero node and channel
+                // (fixed point -> FP32 through an exact double, 2^-kq m for the weights,
+                // 2^(mexp-kq) for the momentum); every entry read non-zero is cleared for the
+                // next block
                 const double unit[2] = {static_cast<double>(__int_as_float((127 - kq) << 23)) * a.mat.mass,
                                         static_cast<double>(__int_as_float((mexp - kq + 127) << 23))};
-                for (int e = tid; e < 8 * kNodesPerBlock; e += THREADS) {
-                    const int o = e >> 7, nd = e & 127;
-                    const int r = WindowOfHalo(o, nd);
-                    if (r < 0) continue;
+                auto flush = [&](int o, int nd, int r) {
                     LdsAcc qv[kMChannels];
                     bool any = false;
 #pragma unroll
@@ -1374,11 +1406,11 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
                         qv[ch] = sM[ch * kMWin + r];
                         any |= qv[ch] != 0;
                     }
-                    if (!any) continue;
+                    if (!any) return;
 #pragma unroll
                     for (int ch = 0; ch < kMChannels; ++ch) sM[ch * kMWin + r] = 0;
                     const uint32_t bi = sHalo[o];
-                    if (bi == kEmpty) continue;
+                    if (bi == kEmpty) return;
                     float* dst = a.M + static_cast<size_t>(bi) * kMFloats + nd;
 #pragma unroll
                     for (int ch = 0; ch < kMChannels; ++ch) {
@@ -1389,15 +1421,34 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
                         const float val = static_cast<float>(d * unit[ch == 0 ? 0 : 1]);
                         if (val != 0.0f) unsafeAtomicAdd(dst + ch * 128, val);
                     }
+                };
+                if (moved) {
+                    // block by block of the neighbourhood
+                    for (int e = tid; e < 8 * kNodesPerBlock; e += THREADS) {
+                        const int r = WindowOfHalo(e >> 7, e & 127);
+                        if (r >= 0) flush(e >> 7, e & 127, r);
+                    }
+                } else {
+                    // no particle left the block's cells 2..5: only nodes [2,6]^3 of grid 0
+                    // and [1,6]^3 of grid 1 hold deposits, 341 of the 1024 above
+                    for (int e = tid; e < kCoreNodes; e += THREADS) {
+                        const bool g1 = e < 216;
+                        const int n = g1 ? 6 : 5, q = g1 ? e : e - 216, lo = g1 ? 1 : 2;
+                        const int lx = (g1 ? q / 36 : q / 25) + lo, qy = g1 ? q / 6 : q / 5;
+                        const int ly = qy - (lx - lo) * n + lo, lz = q - qy * n + lo;
+                        const int r = MEntry(g1 ? 1 : 0, lx, ly, lz);
+                        flush(((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2),
+                              (g1 ? 64 : 0) + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3), r);
+                    }
                 }
             }
             __syncthreads();
             // next round (or block): move totals carried, counts cleared
             for (uint32_t i = tid; i < nch * kHistStride; i += THREADS) sHist[i] = 0;
-            if (tid < kDirections) sRun[tid] += sTot[tid];
+            if (tid < kDirections) sRun[tid] += moved ? sTot[tid] : (tid == 13u ? rn : 0u);
             if (!last) __syncthreads();
         }
-        if (tid < 27) a.cnt[static_cast<size_t>(j) * kDirections + tid] = sRun[tid];
+        if (tid < kDirections) a.cnt[static_cast<size_t>(j) * kDirections + tid] = sRun[tid];
         if (tid == 0) {
             a.blkmax[j] = __uint_as_float(sBlkMax);
             if (sGlobal) atomicAdd(&a.st->p2g_global, sGlobal);

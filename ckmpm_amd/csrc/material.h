@@ -16,6 +16,30 @@ __device__ __forceinline__ void MatMul3(const float (&A)[9], const float (&B)[9]
     for (int i = 0; i < 9; ++i) C[i] = T[i];
 }
 
+// C = A S, S symmetric (xx, xy, xz, yy, yz, zz)
+__device__ __forceinline__ void MatMulSym3(const float (&A)[9], const float (&S)[6], float (&C)[9]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        C[i * 3 + 0] = A[i * 3] * S[0] + A[i * 3 + 1] * S[1] + A[i * 3 + 2] * S[2];
+        C[i * 3 + 1] = A[i * 3] * S[1] + A[i * 3 + 1] * S[3] + A[i * 3 + 2] * S[4];
+        C[i * 3 + 2] = A[i * 3] * S[2] + A[i * 3 + 1] * S[4] + A[i * 3 + 2] * S[5];
+    }
+}
+// k[c][r] = m C_rc - (S T)_rc, S symmetric
+__device__ __forceinline__ void SymMulSub(const float (&S)[6], const float (&T)[9], float m, const float (&C)[9],
+                                          float (&k)[3][3]) {
+    constexpr int kAt[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            float v = m * C[r * 3 + c];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) v = fmaf(-S[kAt[r][q]], T[q * 3 + c], v);
+            k[c][r] = v;
+        }
+}
+
 __device__ __forceinline__ float Det3(const float (&a)[9]) {
     return a[0] * (a[4] * a[8] - a[5] * a[7]) - a[1] * (a[3] * a[8] - a[5] * a[6]) + a[2] * (a[3] * a[7] - a[4] * a[6]);
 }
