@@ -1,0 +1,45 @@
+"""The matrix-function path of the solids' stresses and return maps (polynomials of
+F F^T - I up to a strain norm, the SVD beyond it) against the FP64 oracle: states whose
+strains lie inside, around and beyond the polynomials' ranges.  (Inverted particles of
+moderate F F^T, which only the SVD handles: test_gpu_parity's clamped sand.)"""
+import numpy as np
+import pytest
+
+from ckmpm_amd import scenes
+from ckmpm_amd.engine import engine_from_scene
+from oracle.pyoracle import Oracle
+from tests.test_gpu_parity import GRID_TOL, _box_scene, _grid_close, _import, _rotation
+
+pytestmark = pytest.mark.gpu
+
+
+# |F F^T - I|_F is about 2 sqrt(3) a for the largest stretches 1 +- a: 0.25 (sand, metal) is
+# reached near a = 0.07 and 0.5 (fixed corotated) near a = 0.13
+@pytest.mark.parametrize("kind", [scenes.FIXED_COROTATED, scenes.DRUCKER_PRAGER, scenes.VON_MISES])
+@pytest.mark.parametrize("a", [0.01, 0.07, 0.13, 0.2])
+def test_strain_ranges_lockstep(kind, a):
+    """Singular values in [1 - a, 1 + a], the same a for whole runs of 512 particles and a
+    tenth of it for every other run, so that some wavefronts stay in range and others do
+    not.  Bars as in the stretched-state lockstep test."""
+    sc = _box_scene(kind, seed=81 + kind, speed=0.0)
+    rng = np.random.default_rng(8 + kind)
+    eng = engine_from_scene(sc)
+    orc = Oracle.from_scene(sc)
+    orc.setup()
+    st = eng.state(0)
+    for p in range(st.shape[1]):
+        b = a * (1.0 if (p // 512) % 2 else 0.1)
+        F = _rotation(rng) @ np.diag(rng.uniform(1 - b, 1 + b, 3)) @ _rotation(rng).T
+        st[3:12, p] = (F - np.eye(3)).reshape(9).astype(np.float32)
+    eng.set_state(0, st)
+    for k in range(2):
+        dt = 0.0 if k == 0 else sc.dt
+        _import(eng, orc, 1)
+        orc.physics(dt, sc.dt)
+        eng.Substep(dt, sc.dt)
+        eng.Synchronize()
+        _grid_close(eng.grid_m(), orc.grid_mnext(), GRID_TOL)
+        sg, so = eng.global_state(0), orc.state_next(0)
+        np.testing.assert_allclose(sg[:3], so[:3], rtol=0, atol=2e-7)
+        np.testing.assert_allclose(sg[3:], so[3:], rtol=0, atol=2e-5)
+
