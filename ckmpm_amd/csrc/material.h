@@ -75,15 +75,16 @@ __device__ __forceinline__ float DetIPlusEMinus1(const float (&E)[9]) {
 }
 
 // Isotropic functions of the left strain M = F F^T - I (symmetric, as xx, xy, xz, yy, yz,
-// zz) without its eigenvectors.  The models' stresses and return maps are functions of
-// the principal stretches in the frame of F F^T, i.e. matrix functions f(M): for a
-// polynomial f, the Cayley-Hamilton theorem M^3 = I1 M^2 - I2 M + I3 gives
-// f(M) = a I + b M + c M^2 with scalars from a Horner recurrence of 3 fmas per degree.
-// Where the strain is moderate (|M|_F within the fit's range on every lane of the
-// wavefront, F not inverted), that replaces the SVD and the rebuild from its factors: about
-// 130 instructions instead of 700, on the same data to the same relative precision of the
-// strain.  The coefficients are Chebyshev interpolants of f(m) / m on [-r, r], relative
-// error below 2e-8 in FP32.
+// zz) without its eigenvectors.  A stress that is a function of the principal stretches in
+// the frame of F F^T is a matrix function f(M): for a polynomial f, the Cayley-Hamilton
+// theorem M^3 = I1 M^2 - I2 M + I3 gives f(M) = a I + b M + c M^2 with scalars from a Horner
+// recurrence of 3 fmas per degree.  Where the strain is moderate (|M|_F within the fit's
+// range on every lane of the wavefront, F not inverted) that replaces the SVD: about 130
+// instructions instead of 700, with the same relative precision of the strain.  Two
+// bodies of 15k fixed-corotated particles: 108 -> 101 us per substep.
+// The plastic models keep the SVD: their stored strain follows the rounding of the
+// rebuild U S V^T - I substep by substep, which another route does not reproduce, and
+// their launches gained 0 to 2%.
 struct LeftStrain {
     float M[6], Q[6];  // M and M^2
     float i1, i2, i3;  // invariants of M
@@ -129,17 +130,12 @@ __device__ __forceinline__ void StrainPolynomial(const float (&c)[N + 1], const 
 #pragma unroll
     for (int k = 0; k < 6; ++k) R[k] = fmaf(b, s.M[k], d * s.Q[k]) + ((k == 0 || k == 3 || k == 5) ? a : 0.0f);
 }
-// (1 + m) - sqrt(1 + m) = s (s - 1) on |m| <= 1/2, log(1 + m) / 2 on |m| <= 1/4,
-// exp(x) - 1 on |x| <= 2/5 (all divided by the argument)
-constexpr float kCorotMax = 0.5f, kHenckyMax = 0.25f;
+// s (s - 1) = (1 + m) - sqrt(1 + m), divided by m, on |m| <= 1/2: Chebyshev interpolant,
+// relative error 1.3e-8
+constexpr float kCorotMax = 0.5f;
 __device__ constexpr float kCorotCoef[12] = {5.000000000e-01f,  1.249999925e-01f,  -6.250043213e-02f, 3.906352818e-02f,
                                              -2.732424252e-02f, 2.047590166e-02f,  -1.643312909e-02f, 1.351126283e-02f,
                                              -8.599692956e-03f, 6.669106893e-03f,  -1.521383133e-02f, 1.424708497e-02f};
-__device__ constexpr float kHenckyCoef[9] = {5.000000000e-01f,  -2.499999702e-01f, 1.666665822e-01f,
-                                             -1.250064671e-01f, 1.000099182e-01f,  -8.296582848e-02f,
-                                             7.099088281e-02f,  -7.013241947e-02f, 6.332726777e-02f};
-__device__ constexpr float kExpCoef[7] = {1.000000000e+00f, 5.000000000e-01f, 1.666666716e-01f, 4.166610911e-02f,
-                                          8.333245292e-03f, 1.395849278e-03f, 1.992963371e-04f};
 
 // Every lane's strain lies in the range r of its polynomial, and no lane's F = I + E is
 // inverted (|s_i| >= sqrt(1 - r) then).  Wave-uniform.
@@ -156,32 +152,6 @@ __device__ __forceinline__ void SymToTau(const float (&S)[6], float k, float h, 
     tau[2] = tau[6] = k * S[2];
     tau[5] = tau[7] = k * S[4];
 }
-// F <- (I + Y) F, Y symmetric: E <- E + Y + Y E
-__device__ __forceinline__ void ApplyLeft(const float (&Y)[6], float (&E)[9]) {
-    constexpr int kAt[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
-    float T[9];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            T[i * 3 + j] = Y[kAt[i][j]] + Y[kAt[i][0]] * E[j] + Y[kAt[i][1]] * E[3 + j] + Y[kAt[i][2]] * E[6 + j];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) E[k] += T[k];
-}
-// F <- exp(X) F, X symmetric and small
-__device__ __forceinline__ void ApplyLeftExp(const float (&X)[6], float (&E)[9]) {
-    LeftStrain x;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) x.M[k] = X[k];
-    StrainInvariants(x);
-    float Y[6];
-    StrainPolynomial<6>(kExpCoef, x, Y);
-    ApplyLeft(Y, E);
-}
-__device__ __forceinline__ float FrobeniusSym(const float (&S)[6]) {
-    return sqrtf(S[0] * S[0] + S[3] * S[3] + S[5] * S[5] + 2.0f * (S[1] * S[1] + S[2] * S[2] + S[4] * S[4]));
-}
-
 // Fixed corotated, mpm_material.cuh:318-357: tau = U diag(2 mu s (s - 1) + lambda J (J - 1)) U^T.
 __device__ __forceinline__ void StressFixedCorotated(float lambda, float mu, const float (&E)[9], float (&tau)[9]) {
     LeftStrain ls;
@@ -272,38 +242,6 @@ __device__ __forceinline__ void StressDruckerPrager(float lambda, float mu, floa
                                                     float (&tau)[9]) {
     const float alpha = 0.816496580927726f * 2.0f * sin_phi / (3.0f - sin_phi);  // sqrt(2/3) 2 sin / (3 - sin)
     const float smu = 2.0f * mu;
-    LeftStrain ls;
-    MakeLeftStrain(E, ls);
-    if (StrainInRange(ls, E, kHenckyMax)) {
-        // the same return map on the Hencky strain matrix H = log(F F^T) / 2; every branch
-        // that changes F multiplies it by exp(X), X = H' - H, from the left
-        float H[6], X[6];
-        StrainPolynomial<8>(kHenckyCoef, ls, H);
-        const float hs = H[0] + H[3] + H[5], ht = hs + logJp, third = ht * (1.0f / 3.0f);
-        float D[6] = {H[0] - third, H[1], H[2], H[3] - third, H[4], H[5] - third};
-        bool apply = false;
-        float r = 0.0f;
-        if (ht >= 0.0f) {
-            apply = true;
-            logJp = ht;
-        } else if (mu != 0.0f) {
-            logJp = 0.0f;
-            const float dn = FrobeniusSym(D);
-            const float dg = dn + (3.0f * lambda + smu) / smu * ht * alpha;
-            apply = dg > 0.0f;
-            r = dg / dn;
-        }
-        if (apply) {
-#pragma unroll
-            for (int k = 0; k < 6; ++k) {
-                X[k] = ht >= 0.0f ? -H[k] : -r * D[k];
-                H[k] = ht >= 0.0f ? 0.0f : H[k] + X[k];
-            }
-            ApplyLeftExp(X, E);
-        }
-        SymToTau(H, smu, lambda * (H[0] + H[3] + H[5]), tau);
-        return;
-    }
     Svd3 sv;
     float d[3];
     SignedSvdStrain(E, sv, d);
@@ -408,26 +346,6 @@ __device__ __forceinline__ void PrincipalToTau(const Svd3& sv, const float (&k)[
 // singular values are exp(eps) with the same U, so tau = U diag(2 mu eps + lambda tr eps)
 // U^T directly.
 __device__ __forceinline__ void StressVonMises(float lambda, float mu, float yield, float (&E)[9], float (&tau)[9]) {
-    LeftStrain ls;
-    MakeLeftStrain(E, ls);
-    if (StrainInRange(ls, E, kHenckyMax)) {
-        float H[6], X[6];
-        StrainPolynomial<8>(kHenckyCoef, ls, H);
-        const float tr = H[0] + H[3] + H[5], third = tr * (1.0f / 3.0f);
-        const float D[6] = {H[0] - third, H[1], H[2], H[3] - third, H[4], H[5] - third};
-        const float dn = FrobeniusSym(D), over = dn - yield / (2.0f * mu);
-        if (over > 0.0f && dn > 0.0f) {
-            const float r = over / dn;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) {
-                X[k] = -r * D[k];
-                H[k] += X[k];
-            }
-            ApplyLeftExp(X, E);
-        }
-        SymToTau(H, 2.0f * mu, lambda * tr, tau);
-        return;
-    }
     Svd3 sv;
     float d[3], eps[3];
     SignedSvdStrain(E, sv, d);

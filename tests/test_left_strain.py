@@ -1,7 +1,6 @@
-"""The matrix-function path of the solids' stresses and return maps (polynomials of
-F F^T - I up to a strain norm, the SVD beyond it) against the FP64 oracle: states whose
-strains lie inside, around and beyond the polynomials' ranges.  (Inverted particles of
-moderate F F^T, which only the SVD handles: test_gpu_parity's clamped sand.)"""
+"""Strains inside, around and beyond the range where the fixed-corotated stress is a
+polynomial of F F^T - I (beyond it, and for the plastic models, an SVD) against the FP64
+oracle."""
 import numpy as np
 import pytest
 
@@ -13,8 +12,8 @@ from tests.test_gpu_parity import GRID_TOL, _box_scene, _grid_close, _import, _r
 pytestmark = pytest.mark.gpu
 
 
-# |F F^T - I|_F is about 2 sqrt(3) a for the largest stretches 1 +- a: 0.25 (sand, metal) is
-# reached near a = 0.07 and 0.5 (fixed corotated) near a = 0.13
+# |F F^T - I|_F is up to about 2 sqrt(3) a for stretches in 1 +- a: the polynomial's 0.5 is
+# reached near a = 0.13
 @pytest.mark.parametrize("kind", [scenes.FIXED_COROTATED, scenes.DRUCKER_PRAGER, scenes.VON_MISES])
 @pytest.mark.parametrize("a", [0.01, 0.07, 0.13, 0.2])
 def test_strain_ranges_lockstep(kind, a):
