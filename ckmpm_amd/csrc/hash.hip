@@ -1,12 +1,21 @@
 // Deterministic three-choice bucketed hash of block keys, and its C-ABI.
 //
-// Build (all on the table's stream, no host sync):
+// Build, on the table's stream (6 launches):
+//   1. every pair appends its index to the list of its bucket h_0(key) % B (at most
+//      kListEntries per bucket);
+//   2. per round r: a half wavefront per bucket ranks the bucket's listed pairs by key;
+//      rank < free slots -> slot fill + rank, the rest join their lists of round r + 1;
+//   3. the pairs left after the last round are ranked by key into the stash.
+// The order in which the atomics filled a list does not matter: ranks are by key.  A key
+// set that gives one bucket more than kListEntries pairs (or leaves more than kStashSort)
+// is built instead by sorting (SortedBuild, about 80 launches):
 //   1. sort the (key, value) pairs by key;
 //   2. per round r: bucket[i] = h_r(key_i) % B for unplaced pairs, B (sorts last) for
 //      placed ones; stable sort of pair indices by bucket; rank inside each bucket's
 //      run; pair with rank < free slots of its bucket -> slot fill + rank; then each
 //      run's last element raises the bucket's fill;
 //   3. unplaced pairs, in key order, -> stash.
+// Both builds give the same words.
 // Find: wave-cooperative, a 16-lane quarter wavefront per query and probe (one 8-byte
 // slot per lane, one 128-byte line per bucket), as CooperativeFind
 // (gpu_hash_table.cuh:463-513) does with its 16-thread tiles.
@@ -108,6 +117,112 @@ __global__ void HashStashKernel(const uint32_t* flag, const uint32_t* pos, uint3
         const uint32_t t = *total;
         *nstash = min(t, stash_cap);
         if (t > stash_cap) atomicOr(bad, 4u);
+    }
+}
+
+// Bucket lists of the list build.  A table at its full load has 11.2 pairs per bucket on
+// average in round 0, and a bucket of more than 32 about once in 5 million; later rounds
+// list a few percent of the pairs.  Round r's lists are list[r & 1]: round 2 reuses those
+// of round 0.  All of it lies in the build's temporaries: 67 words per bucket, of at least
+// 11.2 pairs each (6 words a pair), and one word per pair.
+constexpr uint32_t kListEntries = 32;  // half a wavefront
+constexpr uint32_t kStashSort = 1024;
+constexpr uint32_t kBadRebuild = 8u;   // error bit: this key set needs SortedBuild
+struct BucketLists {
+    uint32_t* cnt;   // [3][buckets] pairs that asked for the bucket in each round
+    uint32_t* left;  // pairs left after the last round
+    uint32_t* list;  // [2][buckets][kListEntries] pair indices
+    uint32_t* rest;  // [n] pair indices left after the last round
+    __device__ __forceinline__ void Append(const HashView& h, int r, uint32_t key, uint32_t i) const {
+        const uint32_t b = h.Bucket(key, r);
+        const uint32_t p = atomicAdd(&cnt[static_cast<size_t>(r) * h.buckets + b], 1u);
+        if (p < kListEntries) list[(static_cast<size_t>(r & 1) * h.buckets + b) * kListEntries + p] = i;
+    }
+};
+
+__global__ void HashListClearKernel(BucketLists l, uint32_t buckets, uint32_t* bad, uint32_t* nstash) {
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < kHashRounds * buckets; i += gridDim.x * blockDim.x)
+        l.cnt[i] = 0u;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *l.left = 0u;
+        *bad = 0u;
+        *nstash = 0u;
+    }
+}
+
+__global__ void HashListKernel(HashView h, BucketLists l, const uint32_t* keys, uint32_t n, uint32_t nblocks,
+                               uint32_t* bad) {
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const uint32_t k = keys[i];
+        if (k >= nblocks) atomicOr(bad, 1u);
+        l.Append(h, 0, k, i);
+    }
+}
+
+// Round R: lane l of the 32-lane group holds entry l of the bucket's list; its rank is the
+// number of entries with a smaller (key, index).  Round 0 writes every slot of the table.
+// Bounded by latency (a list, its keys, their atomics: three dependent accesses).  The sort
+// build spent 430 us on 200,003 keys, and 440 us on 25,090 with a 22 us Find of 677k keys,
+// nearly all of it on its 80 launches; this one 64 and 77 (kernels: 40 and 45).
+template <int R>
+__global__ __launch_bounds__(kHashThreads) void HashListPlaceKernel(HashView h, BucketLists l, const uint32_t* keys,
+                                                                    const uint32_t* vals, uint32_t* fill,
+                                                                    uint64_t* slots, uint32_t* bad) {
+    const uint32_t lane = threadIdx.x & 31u;
+    const uint32_t groups = gridDim.x * (kHashThreads / 32);
+    for (uint32_t b = blockIdx.x * (kHashThreads / 32) + (threadIdx.x >> 5); b < h.buckets; b += groups) {
+        const uint32_t c = l.cnt[static_cast<size_t>(R) * h.buckets + b];
+        if (R > 0 && c == 0u) continue;
+        if (c > kListEntries) {
+            if (lane == 0) atomicOr(bad, kBadRebuild);
+            continue;
+        }
+        const uint32_t f = R == 0 ? 0u : fill[b];
+        const bool have = lane < c;
+        const uint32_t i = have ? l.list[(static_cast<size_t>(R & 1) * h.buckets + b) * kListEntries + lane] : 0u;
+        const uint32_t key = have ? keys[i] : 0u, val = have ? vals[i] : 0u;
+        uint32_t rank = 0;
+        bool dup = false;
+        for (uint32_t j = 0; j < c; ++j) {
+            const uint32_t kj = __shfl(key, static_cast<int>(j), 32), ij = __shfl(i, static_cast<int>(j), 32);
+            rank += kj < key || (kj == key && ij < i) ? 1u : 0u;
+            dup |= kj == key && ij != i;
+        }
+        uint64_t* row = slots + static_cast<size_t>(b) * kHashBucket;
+        if (R == 0 && lane >= c && lane < static_cast<uint32_t>(kHashBucket)) row[lane] = kHashEmpty;
+        if (lane == 0) fill[b] = min(static_cast<uint32_t>(kHashBucket), f + c);
+        if (!have) continue;
+        if (dup) atomicOr(bad, 2u);
+        if (rank < kHashBucket - f) row[f + rank] = (static_cast<uint64_t>(key) << 32) | static_cast<uint64_t>(val);
+        else if (R + 1 < kHashRounds) l.Append(h, R + 1, key, i);
+        else l.rest[atomicAdd(l.left, 1u)] = i;
+    }
+}
+
+// One workgroup: thread t ranks pair t of the rest.
+__global__ __launch_bounds__(kStashSort) void HashListStashKernel(BucketLists l, const uint32_t* keys,
+                                                                  const uint32_t* vals, uint64_t* stash,
+                                                                  uint32_t stash_cap, uint32_t* nstash, uint32_t* bad) {
+    __shared__ uint32_t sKey[kStashSort], sIdx[kStashSort];
+    const uint32_t n = *l.left, t = threadIdx.x;
+    if (n > kStashSort) {
+        if (t == 0) atomicOr(bad, kBadRebuild);
+        return;
+    }
+    uint32_t i = 0, key = 0;
+    if (t < n) {
+        sIdx[t] = i = l.rest[t];
+        sKey[t] = key = keys[i];
+    }
+    __syncthreads();
+    if (t < n) {
+        uint32_t rank = 0;
+        for (uint32_t j = 0; j < n; ++j) rank += sKey[j] < key || (sKey[j] == key && sIdx[j] < i) ? 1u : 0u;
+        if (rank < stash_cap) stash[rank] = (static_cast<uint64_t>(key) << 32) | static_cast<uint64_t>(vals[i]);
+    }
+    if (t == 0) {
+        *nstash = min(n, stash_cap);
+        if (n > stash_cap) atomicOr(bad, 4u);
     }
 }
 
@@ -328,8 +443,27 @@ BuildMem MemOf(const ckmpm_hash* h) {
     return b;
 }
 
-// Enqueue the build from device arrays; no host sync.
+// Enqueue the list build from device arrays; no host sync.
 void EnqueueBuild(const BuildMem& b, const uint32_t* keys, const uint32_t* vals, uint32_t n, hipStream_t s) {
+    const uint32_t buckets = b.v.buckets;
+    BucketLists l;
+    l.cnt = b.tmp;
+    l.left = l.cnt + static_cast<size_t>(kHashRounds) * buckets;
+    l.list = l.left + 1;
+    l.rest = l.list + 2ull * kListEntries * buckets;
+    HashListClearKernel<<<LaunchBlocks(kHashRounds * static_cast<uint64_t>(buckets)), kHashThreads, 0, s>>>(
+        l, buckets, b.bad, b.nstash);
+    if (n) HashListKernel<<<LaunchBlocks(n), kHashThreads, 0, s>>>(b.v, l, keys, n, b.nblocks, b.bad);
+    const uint32_t g = LaunchBlocks(32ull * buckets);
+    HashListPlaceKernel<0><<<g, kHashThreads, 0, s>>>(b.v, l, keys, vals, b.fill, b.slots, b.bad);
+    if (n == 0) return;
+    HashListPlaceKernel<1><<<g, kHashThreads, 0, s>>>(b.v, l, keys, vals, b.fill, b.slots, b.bad);
+    HashListPlaceKernel<2><<<g, kHashThreads, 0, s>>>(b.v, l, keys, vals, b.fill, b.slots, b.bad);
+    HashListStashKernel<<<1, kStashSort, 0, s>>>(l, keys, vals, b.stash, b.stash_cap, b.nstash, b.bad);
+}
+
+// Enqueue the sort build (any key set); no host sync.
+void SortedBuild(const BuildMem& b, const uint32_t* keys, const uint32_t* vals, uint32_t n, hipStream_t s) {
     const uint32_t m = b.max_keys;
     uint32_t* t = b.tmp;
     uint32_t *sk = t, *sv = t + m, *placed = t + 2 * m, *bucket = t + 3 * m, *idx = t + 4 * m;
@@ -356,25 +490,33 @@ void EnqueueBuild(const BuildMem& b, const uint32_t* keys, const uint32_t* vals,
     HashStashKernel<<<g, kHashThreads, 0, s>>>(t0, t1, n, sk, sv, b.stash, b.stash_cap, total, b.nstash, b.bad);
 }
 
-// Waits for the build and turns its error bits into a status code (and message).
-int BuildStatus(const uint32_t* bad_dev, hipStream_t s, std::string* err) {
-    uint32_t bad = 0;
-    hipError_t e = hipMemcpyAsync(&bad, bad_dev, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
+// Reads the error bits of the build (waits for it).
+int ReadBad(const uint32_t* bad_dev, uint32_t* bad, hipStream_t s, std::string* err) {
+    hipError_t e = hipMemcpyAsync(bad, bad_dev, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) {
-        if (err) *err = std::string("hash build: ") + hipGetErrorString(e);
-        return CKMPM_ERR_HIP;
+    if (e == hipSuccess) return CKMPM_OK;
+    if (err) *err = std::string("hash build: ") + hipGetErrorString(e);
+    return CKMPM_ERR_HIP;
+}
+
+// Waits for the build, repeats it by sorting where the lists did not hold the key set, and
+// turns the error bits into a status code (and message).
+int FinishBuild(const BuildMem& b, const uint32_t* keys, const uint32_t* vals, uint32_t n, hipStream_t s,
+                std::string* err) {
+    uint32_t bad = 0;
+    int rc = ReadBad(b.bad, &bad, s, err);
+    if (rc == CKMPM_OK && (bad & kBadRebuild)) {
+        SortedBuild(b, keys, vals, n, s);
+        rc = ReadBad(b.bad, &bad, s, err);
     }
+    if (rc != CKMPM_OK) return rc;
     const char* msg = nullptr;
-    int rc = CKMPM_OK;
     if (bad & 1u) msg = "key outside the domain", rc = CKMPM_ERR_INVALID;
     else if (bad & 2u) msg = "duplicate key", rc = CKMPM_ERR_INVALID;
     else if (bad & 4u) msg = "hash stash overflow (too many keys for the table)", rc = CKMPM_ERR_CAPACITY;
     if (msg && err) *err = msg;
     return rc;
 }
-
-int CheckBuild(ckmpm_hash* h) { return BuildStatus(h->bad, h->stream, &h->err); }
 
 // Scratch of the build that allocates nothing (ckmpm_hash_build_noalloc): the
 // temporaries, bucket fills and error word of a table of up to
@@ -445,8 +587,9 @@ int ckmpm_hash_create(const ckmpm_domain_desc* domain, uint32_t max_keys, ckmpm_
 int ckmpm_hash_build_device(ckmpm_hash* h, const uint32_t* keys, const uint32_t* values, uint32_t n) {
     if (!h || (n && (!keys || !values))) return CKMPM_ERR_INVALID;
     if (n > h->max_keys) return HashFail(h, CKMPM_ERR_CAPACITY, "more keys than the table was created for");
-    EnqueueBuild(MemOf(h), keys, values, n, h->stream);
-    return CheckBuild(h);
+    const BuildMem b = MemOf(h);
+    EnqueueBuild(b, keys, values, n, h->stream);
+    return FinishBuild(b, keys, values, n, h->stream, &h->err);
 }
 
 int ckmpm_hash_build_noalloc(const ckmpm_domain_desc* domain, uint32_t max_keys, const uint32_t* keys,
@@ -484,7 +627,7 @@ int ckmpm_hash_build_noalloc(const ckmpm_domain_desc* domain, uint32_t max_keys,
     const hipStream_t s = static_cast<hipStream_t>(stream);
     EnqueueBuild(b, keys, values, n, s);
     if (hipGetLastError() != hipSuccess) return CKMPM_ERR_HIP;
-    return BuildStatus(b.bad, s, nullptr);
+    return FinishBuild(b, keys, values, n, s, nullptr);
 }
 
 int ckmpm_hash_build(ckmpm_hash* h, const uint32_t* keys, const uint32_t* values, uint32_t n) {
@@ -496,8 +639,9 @@ int ckmpm_hash_build(ckmpm_hash* h, const uint32_t* keys, const uint32_t* values
         HASH_HIP(h, hipMemcpyAsync(dk, keys, sizeof(uint32_t) * n, hipMemcpyHostToDevice, h->stream));
         HASH_HIP(h, hipMemcpyAsync(dv, values, sizeof(uint32_t) * n, hipMemcpyHostToDevice, h->stream));
     }
-    EnqueueBuild(MemOf(h), dk, dv, n, h->stream);
-    return CheckBuild(h);
+    const BuildMem b = MemOf(h);
+    EnqueueBuild(b, dk, dv, n, h->stream);
+    return FinishBuild(b, dk, dv, n, h->stream, &h->err);
 }
 
 int ckmpm_hash_find_device(ckmpm_hash* h, const uint32_t* keys, uint32_t n, uint32_t* values, int32_t cooperative) {
