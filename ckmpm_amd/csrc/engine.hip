@@ -165,13 +165,21 @@ void PhaseParticles(ckmpm_engine* e, double dt, double next_dt, FusedRec* rec = 
     // 1-2% (0.25: no more); the single-model 1M jelly lost 12% (one engine in a graph).
     const bool side_by_side = e->models.size() > 1 || (rec && rec->shared);
     const uint32_t grid = GridFor((side_by_side ? e->a_hint / 2u : e->a_hint + e->a_hint / 4u) + 8u);
-    // The models' launches run one after the other on the engine stream.  Running the
-    // second model's on a second stream, concurrently with the first (the launches are
-    // independent; their grid deposits are commutative atomic adds), measured slower on
-    // the 8M fluid + sand scene: 0.614 against 0.607 ms.
+    // Plain calls advance the models of one workgroup size in one launch (G2P2GSet): the
+    // launches are independent (their grid deposits are commutative atomic adds), and one
+    // after the other each leaves a small scene's chip half empty.  Two elastic bodies of
+    // 16k particles: 111 to 81 us per substep; fluid and sand of 73k each: 155 to 127.
+    // Recorded launches stay separate: a graph runs them on queues of their own, which
+    // overlaps different kinds better than one launch does (the 8M fluid + sand scene: 436
+    // against 461 us).  The autotuner times each model alone.
+    const bool tune = e->tuning && !rec;
+    G2P2GSet set[2];
+    set[0].n = set[1].n = 0;
     for (size_t mi = 0; mi < e->models.size(); ++mi) {
         ModelBuf& m = e->models[mi];
-        G2P2GArgs a{};
+        const int t = m.threads == 512 ? 1 : 0;
+        G2P2GArgs& a = set[t].a[set[t].n++];
+        a = G2P2GArgs{};
         a.dom = e->dom;
         a.mat = m.mat;
         a.keys = C.keys;
@@ -196,10 +204,15 @@ void PhaseParticles(ckmpm_engine* e, double dt, double next_dt, FusedRec* rec = 
         a.slot = static_cast<int>(e->substeps & 1u);
         a.blkmax = m.blkmax;
         AdjointIdBuffers(e, mi, &a.ids_in, &a.ids_out);
-        const bool tune = e->tuning && !rec;
+        if (!tune && !rec) continue;
         if (tune) (void)hipEventRecord(m.tune_ev[0], s);
-        Run(rec, kStG2P2G, kFkG2P2G, m.mat.kind * 2 + (m.threads == 512 ? 1 : 0), a, G2P2GGrid(grid), s);
+        Run(rec, kStG2P2G, kFkG2P2G, m.mat.kind * 2 + t, a, G2P2GGrid(grid), s);
         if (tune) (void)hipEventRecord(m.tune_ev[1], s);
+        set[t].n = 0;
+    }
+    for (int t = 0; t < 2; ++t) {
+        if (set[t].n == 1) LaunchOne(kFkG2P2G, set[t].a[0].mat.kind * 2 + t, &set[t].a[0], G2P2GGrid(grid), s);
+        else if (set[t].n > 1) LaunchOne(kFkG2P2GSet, t, &set[t], G2P2GGrid(grid) * set[t].n, s);
     }
     Mark(e);
     // ---- rebin: new layout in P (the previous layout's buffers are free now)

@@ -130,6 +130,12 @@ struct G2P2GArgs {
     uint32_t* ids_out;
 };
 
+// Models of one engine advanced by one launch: n times the workgroups of one.
+struct G2P2GSet {
+    G2P2GArgs a[kMaxModels];
+    uint32_t n;
+};
+
 struct RebinModels {
     int nmodels;
     const uint32_t* cnt[kMaxModels];   // [A_cur][27] direction counts per old block
@@ -225,6 +231,7 @@ struct ScatterMarkArgs {
 enum FusedKernel : int {
     kFkGrid = 0,      // variant: custom boundary
     kFkG2P2G,         // variant: kind * 2 + (threads == 512)
+    kFkG2P2GSet,      // several models, not fused; variant: threads == 512
     kFkRebinCount,
     kFkRebinScan,
     kFkRebinScatter,

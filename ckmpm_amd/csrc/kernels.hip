@@ -1007,21 +1007,29 @@ constexpr int kRoundChunks = 12;
 constexpr uint32_t kRoundParticles = kRoundChunks * 64;
 constexpr int kHistStride = 28;  // per chunk: 27 move counts (then prefixes), padded
 
+struct G2P2GShared {
+    alignas(16) LdsAcc M[kMChannels * kMWin];
+    float V[kVChannels * kVWin];
+    uint16_t code[kRoundParticles];             // move | rank in the chunk << 5
+    uint16_t hist[kRoundChunks * kHistStride];  // per chunk and move
+    uint32_t halo[8];
+    uint32_t run[32];   // particles of the block per move before this round
+    uint32_t tot[32];   // particles per move in this round
+    uint32_t blk_max;   // largest deposit bound of the block (FP32 bits)
+    uint32_t moved;     // a particle of the block has left its cells
+    uint32_t global;    // particles of the block deposited with global atomics
+};
+
 // 4 waves per SIMD: LDS (37.2 KiB per workgroup) allows 4 workgroups per CU; this caps
 // the VGPRs at 128
 template <int KIND, int THREADS>
-__device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint32_t ng) {
+__device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint32_t ng, G2P2GShared& sh) {
     constexpr uint32_t kWaves = THREADS / 64;
-    __shared__ float sV[kVChannels * kVWin];
-    __shared__ __align__(16) LdsAcc sM[kMChannels * kMWin];
-    __shared__ uint16_t sCode[kRoundParticles];               // move | rank in the chunk << 5
-    __shared__ uint16_t sHist[kRoundChunks * kHistStride];    // per chunk and move
-    __shared__ uint32_t sHalo[8];
-    __shared__ uint32_t sRun[32];   // particles of the block per move before this round
-    __shared__ uint32_t sTot[32];   // particles per move in this round
-    __shared__ uint32_t sBlkMax;    // largest deposit bound of the block (FP32 bits)
-    __shared__ uint32_t sMoved;     // a particle of the block has left its cells
-    __shared__ uint32_t sGlobal;    // particles of the block deposited with global atomics
+    float* const sV = sh.V;
+    LdsAcc* const sM = sh.M;
+    uint16_t *const sCode = sh.code, *const sHist = sh.hist;
+    uint32_t *const sHalo = sh.halo, *const sRun = sh.run, *const sTot = sh.tot;
+    uint32_t &sBlkMax = sh.blk_max, &sMoved = sh.moved, &sGlobal = sh.global;
 
     const uint32_t A = a.lc->A, Nb = a.lc->Nb;
     const uint32_t tid = threadIdx.x, lane = LaneId(), wave = tid >> 6;
@@ -1464,7 +1472,30 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     using CT = const __attribute__((address_space(4))) G2P2GArgs;
     CT* p = (CT*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(p));
-    G2P2GBody<KIND, THREADS>(*(const G2P2GArgs*)p, blockIdx.x, gridDim.x);
+    __shared__ G2P2GShared sh;
+    G2P2GBody<KIND, THREADS>(*(const G2P2GArgs*)p, blockIdx.x, gridDim.x, sh);
+}
+
+// Several models of one engine in one launch, one model's workgroups after the other's.
+// The workgroup branches on its model's kind, which is uniform; the bodies share the LDS.
+// (Models taking 8 workgroups in turn: no difference for small scenes, and 520 against 461
+// us for the 8M fluid + sand scene, whose CUs then run both kinds at once.)
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) void G2P2GSetKernel(G2P2GSet s) {
+    using CT = const __attribute__((address_space(4))) G2P2GSet;
+    CT* p = (CT*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    __shared__ G2P2GShared sh;
+    const uint32_t ng = gridDim.x / p->n, m = blockIdx.x / ng, wg = blockIdx.x - m * ng;
+    const G2P2GArgs& a = ((const G2P2GSet*)p)->a[m];
+    switch (a.mat.kind) {
+        case kFixedCorotated: G2P2GBody<kFixedCorotated, THREADS>(a, wg, ng, sh); break;
+        case kNeoHookean: G2P2GBody<kNeoHookean, THREADS>(a, wg, ng, sh); break;
+        case kDruckerPrager: G2P2GBody<kDruckerPrager, THREADS>(a, wg, ng, sh); break;
+        case kVonMises: G2P2GBody<kVonMises, THREADS>(a, wg, ng, sh); break;
+        case kCamClay: G2P2GBody<kCamClay, THREADS>(a, wg, ng, sh); break;
+        default: G2P2GBody<kFluid, THREADS>(a, wg, ng, sh); break;
+    }
 }
 
 // ============================================================== rebin
@@ -1871,6 +1902,12 @@ void LaunchOne(int kernel, int variant, const void* args, uint32_t grid, hipStre
             else LaunchG2P2GT<256>(a, grid, s);
             break;
         }
+        case kFkG2P2GSet: {
+            const auto& a = *static_cast<const G2P2GSet*>(args);
+            if (variant & 1) G2P2GSetKernel<512><<<grid, 512, 0, s>>>(a);
+            else G2P2GSetKernel<256><<<grid, 256, 0, s>>>(a);
+            break;
+        }
         case kFkRebinCount:
             RebinCountKernel<<<grid, kCountThreads, 0, s>>>(*static_cast<const RebinCountArgs*>(args));
             break;
@@ -1931,7 +1968,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     const G2P2GArgs* __restrict__ tab, const uint32_t* __restrict__ begin, uint32_t n) {
     uint32_t wg, ng;
     const uint32_t i = FusedScene(begin, n, wg, ng);
-    G2P2GBody<KIND, THREADS>(FusedArgs(tab, i), wg, ng);
+    __shared__ G2P2GShared sh;
+    G2P2GBody<KIND, THREADS>(FusedArgs(tab, i), wg, ng, sh);
 }
 #define CKMPM_FUSED(NAME, BODY, ARGS, THREADS)                                                                  \
     __global__ __launch_bounds__(THREADS) void NAME(const ARGS* __restrict__ tab, const uint32_t* __restrict__ begin, \
