@@ -143,45 +143,44 @@ __device__ __forceinline__ bool StrainInRange(const LeftStrain& s, const float (
     const float F[9] = {1.0f + E[0], E[1], E[2], E[3], 1.0f + E[4], E[5], E[6], E[7], 1.0f + E[8]};
     return __all(s.qq <= r * r && Det3(F) > 0.0f) != 0;
 }
-// tau (9, symmetric) = k S + h I
-__device__ __forceinline__ void SymToTau(const float (&S)[6], float k, float h, float (&tau)[9]) {
-    tau[0] = fmaf(k, S[0], h);
-    tau[4] = fmaf(k, S[3], h);
-    tau[8] = fmaf(k, S[5], h);
-    tau[1] = tau[3] = k * S[1];
-    tau[2] = tau[6] = k * S[2];
-    tau[5] = tau[7] = k * S[4];
-}
 // Fixed corotated, mpm_material.cuh:318-357: tau = U diag(2 mu s (s - 1) + lambda J (J - 1)) U^T.
 __device__ __forceinline__ void StressFixedCorotated(float lambda, float mu, const float (&E)[9], float (&tau)[9]) {
     LeftStrain ls;
     MakeLeftStrain(E, ls);
+    float T[6];  // tau as xx, xy, xz, yy, yz, zz
     if (StrainInRange(ls, E, kCorotMax)) {
         float S[6];
         StrainPolynomial<11>(kCorotCoef, ls, S);
         // J^2 - 1 = I1 + I2 + I3 of M: as precise as M, which det E and tr E are not once F
         // holds a rotation
         const float w = ls.i1 + ls.i2 + ls.i3, dj = w * __builtin_amdgcn_rcpf(1.0f + sqrtf(1.0f + w));
-        SymToTau(S, 2.0f * mu, lambda * (1.0f + dj) * dj, tau);
-        return;
+        const float k = 2.0f * mu, h = lambda * (1.0f + dj) * dj;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) T[q] = q == 0 || q == 3 || q == 5 ? fmaf(k, S[q], h) : k * S[q];
+    } else {
+        Svd3 sv;
+        float d[3];
+        SignedSvdStrain(E, sv, d);
+        const float jm1 = d[0] + d[1] + d[2] + d[0] * d[1] + d[0] * d[2] + d[1] * d[2] + d[0] * d[1] * d[2];
+        const float vol = lambda * (1.0f + jm1) * jm1;
+        float k[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) k[a] = 2.0f * mu * sv.s[a] * d[a] + vol;
+        int q = 0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = i; j < 3; ++j)
+                T[q++] = sv.U[i * 3 + 0] * k[0] * sv.U[j * 3 + 0] + sv.U[i * 3 + 1] * k[1] * sv.U[j * 3 + 1] +
+                         sv.U[i * 3 + 2] * k[2] * sv.U[j * 3 + 2];
     }
-    Svd3 sv;
-    float d[3];
-    SignedSvdStrain(E, sv, d);
-    const float jm1 = d[0] + d[1] + d[2] + d[0] * d[1] + d[0] * d[2] + d[1] * d[2] + d[0] * d[1] * d[2];
-    const float vol = lambda * (1.0f + jm1) * jm1;
-    float k[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) k[a] = 2.0f * mu * sv.s[a] * d[a] + vol;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = i; j < 3; ++j) {
-            const float v = sv.U[i * 3 + 0] * k[0] * sv.U[j * 3 + 0] + sv.U[i * 3 + 1] * k[1] * sv.U[j * 3 + 1] +
-                            sv.U[i * 3 + 2] * k[2] * sv.U[j * 3 + 2];
-            tau[i * 3 + j] = v;
-            tau[j * 3 + i] = v;
-        }
+    // written once, after the branches: stored in each of them, tau stayed in scratch memory
+    tau[0] = T[0];
+    tau[4] = T[3];
+    tau[8] = T[5];
+    tau[1] = tau[3] = T[1];
+    tau[2] = tau[6] = T[2];
+    tau[5] = tau[7] = T[4];
 }
 
 // log(1 + d) and exp(x) of the small principal strains: for |d|, |x| <= 1/32 their
