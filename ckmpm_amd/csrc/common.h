@@ -51,6 +51,12 @@ struct Status {
     uint32_t dep_bits[2][kMaxModels];
 };
 
+// What the host reads after a substep, in pinned memory.
+struct HostStatus {
+    Status st;
+    LayoutCounts lc;
+};
+
 struct DomainDev {
     int dim[3];
     int off[3];

@@ -19,7 +19,10 @@ using namespace ckmpm;
 
 namespace {
 
-
+// Largest position array staged in pinned host memory for a pageable destination; above it
+// the copy into the user's memory is what counts, and the runtime overlaps its pieces (8k
+// particles: 18 against 25 us or more staged on the device; 97k: 98 against 90).
+constexpr size_t kHostStageBytes = 1ull << 20;
 
 uint32_t GridFor(uint32_t blocks) {
     uint32_t g = std::max<uint32_t>(blocks, 8u);
@@ -36,9 +39,11 @@ int FlagsToCode(uint32_t f) {
 }
 
 int ReadStatus(ckmpm_engine* e, Status& st, LayoutCounts& lc) {
-    CK_HIP(e, hipMemcpyAsync(&st, e->status, sizeof(Status), hipMemcpyDeviceToHost, e->stream));
-    CK_HIP(e, hipMemcpyAsync(&lc, e->L[e->cur].lc, sizeof(LayoutCounts), hipMemcpyDeviceToHost, e->stream));
+    LaunchExportStatus(e->status, e->L[e->cur].lc, e->host_status, e->stream);
+    CK_HIP(e, hipGetLastError());
     CK_HIP(e, hipStreamSynchronize(e->stream));
+    st = e->host_status->st;
+    lc = e->host_status->lc;
     e->a_hint = lc.A;
     return CKMPM_OK;
 }
@@ -261,6 +266,26 @@ int CopyOnStream(ckmpm_engine* e, void* dst, const void* src, size_t bytes, hipM
     return CKMPM_OK;
 }
 
+// The device's address of the host range [p, p + bytes), where all of it lies in one pinned
+// allocation (a kernel can then store to it: one launch in place of a staging launch and a
+// copy behind it, 16 against 26 us for the positions of 8k particles, 235 against 244 for
+// 1M; a plain copy of the state, which needs no launch, is faster as a copy); null for
+// other memory.
+void* PinnedView(void* p, size_t bytes) {
+    hipPointerAttribute_t at{};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    int dev = -1;
+    if (hipGetDevice(&dev) == hipSuccess && hipPointerGetAttributes(&at, p) == hipSuccess &&
+        at.type == hipMemoryTypeHost && at.devicePointer && at.device == dev &&
+        hipMemGetAddressRange(&base, &size, at.devicePointer) == hipSuccess) {
+        const size_t at0 = static_cast<char*>(at.devicePointer) - static_cast<char*>(base);
+        if (at0 <= size && bytes <= size - at0) return at.devicePointer;
+    }
+    (void)hipGetLastError();  // pageable memory is not an error
+    return nullptr;
+}
+
 int CheckReady(ckmpm_engine* e) {
     if (!e) return CKMPM_ERR_INVALID;
     if (!e->setup_done) return Fail(e, CKMPM_ERR_INVALID, "call ckmpm_initial_setup first");
@@ -318,6 +343,8 @@ int ckmpm_create(const ckmpm_domain_desc* domain, const ckmpm_sim_desc* sim, ckm
     check(Alloc(e, &e->word_off, e->nwords));
     check(Alloc(e, &e->total, 4));
     check(Alloc(e, &e->scan_tmp, ScanTempWords(std::max<size_t>(e->cap, e->nwords))));
+    if (rc == CKMPM_OK && hipHostMalloc(reinterpret_cast<void**>(&e->host_status), sizeof(HostStatus), hipHostMallocDefault) != hipSuccess)
+        rc = Fail(e, CKMPM_ERR_HIP, "hipHostMalloc");
     if (rc == CKMPM_OK) {
         for (int i = 0; i < 2; ++i) {
             (void)hipMemsetAsync(e->L[i].table, 0xFF, nblocks * sizeof(uint32_t), e->stream);
@@ -698,17 +725,27 @@ int ckmpm_get_positions(ckmpm_engine* e, int32_t model, float* xyz, uint64_t cap
     if (model < 0 || model >= static_cast<int32_t>(e->models.size()) || !xyz) return CKMPM_ERR_INVALID;
     ModelBuf& m = e->models[model];
     if (capacity < m.n) return Fail(e, CKMPM_ERR_INVALID, "capacity below particle count");
+    const size_t bytes = 3 * sizeof(float) * static_cast<size_t>(m.n);
+    float* direct = static_cast<float*>(PinnedView(xyz, bytes));
     // staging buffer for the largest model, allocated on the first call and kept (a frame
     // loop calls this once per frame)
-    if (!e->pos_stage) {
+    if (!direct && !e->pos_stage && !e->host_stage) {
         uint32_t nmax = 0;
         for (const ModelBuf& q : e->models) nmax = std::max(nmax, q.n);
-        CK_TRY(Alloc(e, &e->pos_stage, 3 * static_cast<size_t>(nmax)));
+        const size_t most = 3 * sizeof(float) * static_cast<size_t>(nmax);
+        if (most <= kHostStageBytes) CK_HIP(e, hipHostMalloc(reinterpret_cast<void**>(&e->host_stage), most, hipHostMallocDefault));
+        else CK_TRY(Alloc(e, &e->pos_stage, 3 * static_cast<size_t>(nmax)));
     }
+    float* dst = direct ? direct : (e->host_stage ? e->host_stage : e->pos_stage);
     const LayoutBuf& P = e->L[1 - e->cur];
-    LaunchExportPositions(e->dom, P.keys, P.lc, m.off[1 - e->sc], m.st[e->sc], m.n, e->pos_stage,
-                          GridFor(e->a_hint + 8), e->stream);
-    CK_TRY(CopyOnStream(e, xyz, e->pos_stage, 3 * sizeof(float) * static_cast<size_t>(m.n), hipMemcpyDeviceToHost));
+    LaunchExportPositions(e->dom, P.keys, P.lc, m.off[1 - e->sc], m.st[e->sc], m.n, dst, GridFor(e->a_hint + 8), e->stream);
+    if (dst == e->pos_stage) {
+        CK_TRY(CopyOnStream(e, xyz, dst, bytes, hipMemcpyDeviceToHost));
+    } else {
+        CK_HIP(e, hipGetLastError());
+        CK_HIP(e, hipStreamSynchronize(e->stream));
+        if (dst == e->host_stage) std::memcpy(xyz, dst, bytes);
+    }
     if (n) *n = m.n;
     return CKMPM_OK;
 }
@@ -820,6 +857,8 @@ int ckmpm_destroy(ckmpm_engine* e) {
         for (hipEvent_t ev : m.tune_ev)
             if (ev) (void)hipEventDestroy(ev);
     for (void* p : e->allocs) (void)hipFree(p);
+    if (e->host_status) (void)hipHostFree(e->host_status);
+    if (e->host_stage) (void)hipHostFree(e->host_stage);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
     return CKMPM_OK;

@@ -79,7 +79,11 @@ struct ckmpm_engine {
     uint32_t* tsum = nullptr;         // rebin count tile sums
     uint32_t* scan_tmp = nullptr;
     uint32_t* total = nullptr;
-    float* pos_stage = nullptr;  // ckmpm_get_positions staging (3 floats per particle of the largest model)
+    HostStatus* host_status = nullptr;  // pinned: status and block counts of the last host read
+    // ckmpm_get_positions staging of 3 floats per particle of the largest model: in pinned
+    // host memory up to kHostStageBytes, in device memory for a larger model
+    float* host_stage = nullptr;
+    float* pos_stage = nullptr;
     std::vector<ModelBuf> models;
     int sc = 0;           // state / ordering buffer index of the current step
     bool setup_done = false;

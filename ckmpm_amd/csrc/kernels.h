@@ -52,6 +52,8 @@ void LaunchInitState(const DomainDev& d, int kind, const float* xyz, const float
                      uint64_t rigid_count = 0);
 void LaunchExportPositions(const DomainDev& d, const uint32_t* keys, const LayoutCounts* lc, const uint32_t* off,
                            const float* st, uint32_t n, float* xyz, uint32_t grid, hipStream_t s);
+// Status and block counts into pinned host memory, complete once the stream is synchronised.
+void LaunchExportStatus(const Status* st, const LayoutCounts* lc, HostStatus* out, hipStream_t s);
 void LaunchRasterize(const DomainDev& d, const float* xyz, const float* vel, uint32_t n, uint32_t nvel, float mass,
                      const uint32_t* table, const LayoutCounts* lc, float* M, Status* st, hipStream_t s);
 

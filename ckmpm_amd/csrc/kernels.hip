@@ -375,20 +375,39 @@ __global__ void RasterizeKernel(DomainDev d, const float* xyz, const float* vel,
 }
 
 // Global positions of the stored state: slot t was written while processing block j of
-// the previous ordering (off_prev), relative to that block's origin.
+// the previous ordering (off_prev), relative to that block's origin.  The rows of 256
+// particles go through LDS so that a wavefront stores 256 contiguous bytes: xyz may be host
+// memory, where every store crosses the bus.
 __global__ __launch_bounds__(kThreads) void ExportPositionsKernel(DomainDev d, const uint32_t* keys,
                                                                   const LayoutCounts* lc, const uint32_t* off,
                                                                   const float* st, uint32_t n, float* xyz) {
+    __shared__ float row[3 * kThreads];
     const uint32_t A = lc->A;
     const size_t N = n;
     for (uint32_t j = blockIdx.x; j < A; j += gridDim.x) {
         int b[3];
         CoordsOf(d, keys[j], b[0], b[1], b[2]);
-        for (uint32_t t = off[j] + threadIdx.x; t < off[j + 1] && t < n; t += kThreads)
+        const uint32_t end = min(off[j + 1], n);
+        for (uint32_t t0 = off[j]; t0 < end; t0 += kThreads) {
+            const uint32_t t = t0 + threadIdx.x, m = min(end - t0, static_cast<uint32_t>(kThreads));
+            if (t < end)
 #pragma unroll
-            for (int k = 0; k < 3; ++k)
-                xyz[3 * static_cast<size_t>(t) + k] = __fadd_rn(__fmul_rn(static_cast<float>(4 * b[k]), d.dx), st[k * N + t]);
+                for (int k = 0; k < 3; ++k)
+                    row[3 * threadIdx.x + k] = __fadd_rn(__fmul_rn(static_cast<float>(4 * b[k]), d.dx), st[k * N + t]);
+            __syncthreads();
+            float* dst = xyz + 3 * static_cast<size_t>(t0);
+            for (uint32_t i = threadIdx.x; i < 3 * m; i += kThreads) dst[i] = row[i];
+            __syncthreads();
+        }
     }
+}
+
+// Status and block counts into the host's copy.
+__global__ void ExportStatusKernel(const Status* st, const LayoutCounts* lc, HostStatus* out) {
+    const uint32_t i = threadIdx.x;
+    uint32_t* dst = reinterpret_cast<uint32_t*>(out);
+    if (i < sizeof(Status) / 4) dst[i] = reinterpret_cast<const uint32_t*>(st)[i];
+    else if (i < sizeof(HostStatus) / 4) dst[i] = reinterpret_cast<const uint32_t*>(lc)[i - sizeof(Status) / 4];
 }
 
 // ============================================================== layout kernels
@@ -1847,6 +1866,10 @@ void LaunchInitState(const DomainDev& d, int kind, const float* xyz, const float
 void LaunchExportPositions(const DomainDev& d, const uint32_t* keys, const LayoutCounts* lc, const uint32_t* off,
                            const float* st, uint32_t n, float* xyz, uint32_t grid, hipStream_t s) {
     ExportPositionsKernel<<<grid, kThreads, 0, s>>>(d, keys, lc, off, st, n, xyz);
+}
+void LaunchExportStatus(const Status* st, const LayoutCounts* lc, HostStatus* out, hipStream_t s) {
+    static_assert(sizeof(HostStatus) == sizeof(Status) + sizeof(LayoutCounts) && sizeof(HostStatus) <= 4 * 64, "a word per lane");
+    ExportStatusKernel<<<1, 64, 0, s>>>(st, lc, out);
 }
 void LaunchRasterize(const DomainDev& d, const float* xyz, const float* vel, uint32_t n, uint32_t nvel, float mass,
                      const uint32_t* table, const LayoutCounts* lc, float* M, Status* st, hipStream_t s) {
