@@ -28,7 +28,15 @@
 
 namespace {
 
-constexpr int kAT = 256;         // threads per workgroup
+// Threads per workgroup of the particle backward.  The registers allow 8 wavefronts per CU:
+// as four workgroups of two, with a block's particles split over several, all of a small
+// scene's chunks run at once (104k fixed-corotated particles in 320 blocks: 47.8 us per
+// launch, 50.1 as two workgroups of four).  What bounds it there is the chain of memory
+// latencies (about 60% of a wavefront's cycles) and 3800 vector instructions per chunk;
+// element loads of whole 8^3 windows, 48 of them in a row, had taken it to 56.7 (9k
+// Neo-Hookean: 38.5, now 28.6).
+constexpr int kBT = 128;
+constexpr int kAT = 256;         // threads per workgroup of the other kernels
 constexpr int kAWin = 512;       // 8^3 nodes of one sub-grid window
 
 uint32_t AGrid(uint64_t n) {
@@ -177,7 +185,28 @@ struct AdjArgs {
     uint32_t cap;
 };
 
-__device__ __forceinline__ float W0p(float t) { return -1.0f + cospif(2.0f * t); }
+// Slopes d w0 / d t = -1 + cos(2 pi t) of both sub-grids, one cosine per axis: the grids'
+// offsets differ by 1/2, so their cosines by the sign.  With f = min(t0, t1) in [0, 1/2) and
+// f' = min(f, 1/2 - f) in [0, 1/4], cos(2 pi f) = +-cos(2 pi f'), where the Taylor series
+// through x^12 is within 7e-9 (the next term, x^14 / 14!, at x = pi / 2).
+__device__ __forceinline__ void StencilSlopes(const Stencil32 (&s)[2], float (&dw)[2][3]) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const float f = fminf(s[0].t[a], s[1].t[a]);
+        const float g = 0.5f - f, fp = fminf(f, g);
+        const float z = 39.47841760435743f * fp * fp;  // (2 pi f')^2
+        float p = 2.087675698786810e-09f;              //  1 / 12!
+        p = fmaf(p, z, -2.755731922398589e-07f);       // -1 / 10!
+        p = fmaf(p, z, 2.480158730158730e-05f);        //  1 / 8!
+        p = fmaf(p, z, -1.388888888888889e-03f);       // -1 / 6!
+        p = fmaf(p, z, 4.166666666666666e-02f);        //  1 / 4!
+        p = fmaf(p, z, -0.5f);
+        p = fmaf(p, z, 1.0f);
+        const float c = (g < f) != (s[0].t[a] >= 0.5f) ? -p : p;  // cos(2 pi t0)
+        dw[0][a] = c - 1.0f;
+        dw[1][a] = -1.0f - c;
+    }
+}
 
 // Gradient (w.r.t. the position, per axis) of the node-(ox,oy,oz) weight.
 __device__ __forceinline__ void WeightGrad(const Stencil32& s, const float (&dw)[3], int ox, int oy, int oz,
@@ -212,6 +241,16 @@ __device__ __forceinline__ void MomentAdjoint(const Stencil32& s, const float (&
     }
 }
 
+// a (9) = k s, s symmetric as xx, xy, xz, yy, yz, zz
+__device__ __forceinline__ void Unpack(const float (&s)[6], float k, float (&a)[9]) {
+    a[0] = k * s[0];
+    a[1] = a[3] = k * s[1];
+    a[2] = a[6] = k * s[2];
+    a[4] = k * s[3];
+    a[5] = a[7] = k * s[4];
+    a[8] = k * s[5];
+}
+
 __device__ __forceinline__ void Cofactor(const float (&F)[9], float (&c)[9]) {
     c[0] = F[4] * F[8] - F[5] * F[7];
     c[1] = F[5] * F[6] - F[3] * F[8];
@@ -226,11 +265,13 @@ __device__ __forceinline__ void Cofactor(const float (&F)[9], float (&c)[9]) {
 
 // 2 waves per SIMD: 256 VGPRs (a few spills for FC) instead of ~275 and one wave
 template <int KIND>
-__global__ __launch_bounds__(kAT) __attribute__((amdgpu_waves_per_eu(2, 2))) void G2P2GBackwardKernel(AdjArgs a) {
-    __shared__ float sV[kVChannels * 2 * kAWin];
-    __shared__ float sMb[kMChannels * 2 * kAWin];
-    __shared__ double sVb[kVChannels * 2 * kAWin];
+__global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(2, 2))) void G2P2GBackwardKernel(AdjArgs a) {
+    __shared__ float sV[kVChannels * kVWin];
+    __shared__ __align__(16) float sMb[kMChannels * 2 * kAWin];
+    __shared__ __align__(16) double sVb[kVChannels * kVWin + 1];  // the velocity window's adjoint
     __shared__ uint32_t sHalo[8];
+    // the adjoints wait until the SVD is done: held across it, they spill 14 VGPRs
+    constexpr bool kEarly = KIND != kFixedCorotated;
     const uint32_t A = a.lc->A, Nb = a.lc->Nb;
     const uint32_t tid = threadIdx.x;
     const float dx = a.dom.dx, inv_dx = a.dom.inv_dx;
@@ -238,14 +279,48 @@ __global__ __launch_bounds__(kAT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const float mass = a.mat.mass;
     if (a.Mzero) {
         const size_t nz = static_cast<size_t>(min(a.lc_zero->Nb, a.cap)) * kMFloats;
-        for (size_t i = blockIdx.x * static_cast<size_t>(kAT) + tid; i < nz; i += static_cast<size_t>(gridDim.x) * kAT)
+        for (size_t i = blockIdx.x * static_cast<size_t>(kBT) + tid; i < nz; i += static_cast<size_t>(gridDim.x) * kBT)
             a.Mzero[i] = 0.0f;
     }
     // workgroup w serves part w % split of blocks w / split, w / split + gridDim / split, ...
     const uint32_t part = blockIdx.x % a.split, per = gridDim.x / a.split;
     for (uint32_t j = blockIdx.x / a.split; j < A; j += per) {
         const uint32_t beg = a.off[j], end = a.off[j + 1];
-        if (beg + part * kAT >= end) continue;  // no chunk for this part
+        if (beg + part * kBT >= end) continue;  // no chunk for this part
+        // A chunk's inputs are requested before the halo (the first chunk's) or at the end of
+        // the chunk before, so that they arrive while other work runs.
+        uint32_t t = beg + part * kBT + tid, s = 0;
+        float x[3], E[9], lam = a.mat.lambda, mu = a.mat.mu, xbn[3], Fb[9], lamb = 0.0f, mub = 0.0f;
+        auto load_adjoints = [&]() {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) xbn[k] = a.xb_in[k * N + t];
+#pragma unroll
+            for (int k = 0; k < 9; ++k) Fb[k] = a.Eb_in[k * N + t];
+            lamb = a.tb_in[t];
+            mub = a.tb_in[N + t];
+        };
+        auto load = [&]() {
+            if (t >= end) return;
+            const uint32_t pe = a.perm[t];
+            s = pe & kSlotMask;
+            int mvv = static_cast<int>(pe >> kMoveShift);
+            if (s >= a.n || mvv >= kDirections) {
+                s = 0;
+                mvv = 13;
+            }
+            const int mov[3] = {mvv / 9 - 1, (mvv / 3) % 3 - 1, mvv % 3 - 1};
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                x[k] = __fsub_rn(a.st_in[k * N + s], __fmul_rn(static_cast<float>(4 * mov[k]), dx));
+#pragma unroll
+            for (int k = 0; k < 9; ++k) E[k] = a.st_in[(3 + k) * N + s];
+            if (a.pp_attr) {
+                lam = a.st_in[a.pp_attr * N + s];
+                mu = a.st_in[(a.pp_attr + 1) * N + s];
+            }
+            if (kEarly) load_adjoints();
+        };
+        load();
         int bb[3];
         CoordsOf(a.dom, a.keys[j], bb[0], bb[1], bb[2]);
         if (tid < 8) {
@@ -255,101 +330,60 @@ __global__ __launch_bounds__(kAT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             if (bi != kEmpty && bi >= Nb) bi = kEmpty;
             sHalo[tid] = bi;
         }
-        for (int i = tid; i < kVChannels * 2 * kAWin; i += kAT) sVb[i] = 0.0;
+        for (int i = 2 * tid; i < kVChannels * kVWin; i += 2 * kBT)
+            *reinterpret_cast<uint4*>(sVb + i) = make_uint4(0u, 0u, 0u, 0u);
         __syncthreads();
-        for (int i = tid; i < 8 * kMFloats; i += kAT) {
-            const int o = i / kMFloats, r = i % kMFloats;
-            const int ch = r >> 7, node = r & 127, g = node >> 6;
-            const int lx = ((node >> 4) & 3) + 4 * ((o >> 2) & 1);
-            const int ly = ((node >> 2) & 3) + 4 * ((o >> 1) & 1);
-            const int lz = (node & 3) + 4 * (o & 1);
-            const uint32_t bi = sHalo[o];
-            const int l = (ch * 2 + g) * kAWin + lx * 64 + ly * 8 + lz;
-            sMb[l] = bi != kEmpty ? a.Mbar[static_cast<size_t>(bi) * kMFloats + r] : 0.0f;
-            if (ch < 3) sV[l] = bi != kEmpty ? a.V[static_cast<size_t>(bi) * kVFloats + r] : 0.0f;
+        // halo: the velocity window, and M-bar over the whole 8^3 window as 16-byte loads of a
+        // z column of a grid block, all of them in flight
+        StageVelocity<kBT>(sV, a.V, sHalo, tid);
+        {
+            constexpr int kPer = 8 * kMFloats / 4 / kBT;
+            static_assert(kPer * kBT * 4 == 8 * kMFloats && kMFloats / 4 == kBT, "a block per pass");
+            float4 q[kPer];
+#pragma unroll
+            for (int o = 0; o < kPer; ++o) {
+                const uint32_t bi = sHalo[o];
+                const float4* src = reinterpret_cast<const float4*>(a.Mbar + static_cast<size_t>(bi) * kMFloats);
+                q[o] = bi != kEmpty ? src[tid] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+            // column tid = ch * 32 + g * 16 + x * 4 + y of block o
+            const int l0 = (tid >> 4) * kAWin + ((tid >> 2) & 3) * 64 + (tid & 3) * 8;
+#pragma unroll
+            for (int o = 0; o < kPer; ++o)
+                *reinterpret_cast<float4*>(sMb + l0 + ((o >> 2) & 1) * 256 + ((o >> 1) & 1) * 32 + (o & 1) * 4) = q[o];
         }
         __syncthreads();
-        for (uint32_t c0 = beg + part * kAT; c0 < end; c0 += a.split * kAT) {
-            const uint32_t t = c0 + tid;
+        for (uint32_t c0 = beg + part * kBT; c0 < end; c0 += a.split * kBT) {
             if (t < end) {
-                const uint32_t pe = a.perm[t];
-                uint32_t s = pe & kSlotMask;
-                int mvv = static_cast<int>(pe >> kMoveShift);
-                if (s >= a.n || mvv >= kDirections) {
-                    s = 0;
-                    mvv = 13;
-                }
-                const int mov[3] = {mvv / 9 - 1, (mvv / 3) % 3 - 1, mvv % 3 - 1};
-                float x[3], E[9];
-#pragma unroll
-                for (int k = 0; k < 3; ++k)
-                    x[k] = __fsub_rn(a.st_in[k * N + s], __fmul_rn(static_cast<float>(4 * mov[k]), dx));
-#pragma unroll
-                for (int k = 0; k < 9; ++k) E[k] = a.st_in[(3 + k) * N + s];
-                float lam = a.mat.lambda, mu = a.mat.mu;
-                if (a.pp_attr) {
-                    lam = a.st_in[a.pp_attr * N + s];
-                    mu = a.st_in[(a.pp_attr + 1) * N + s];
-                }
                 // ======================= forward recompute (as G2P2GKernel)
                 float xs[3];
 #pragma unroll
                 for (int k = 0; k < 3; ++k) xs[k] = __fmul_rn(x[k], inv_dx);
                 Stencil32 sp[2];
-                MakeStencilPair(xs, sp[0], sp[1]);
-                int lw[2][3];
-                float v[3] = {0.f, 0.f, 0.f}, B[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                float D[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                float s6[6], msn[3], mdg[3];  // a symmetric matrix, the moments of the stencils
+                // base cells 2..5, as the forward takes them; a position farther out (an
+                // imported state) reads and scatters the grid blocks themselves
+                MakeStencilPair<2, 5>(xs, sp[0], sp[1], msn, mdg);
+                float v[3], B[9];  // v: sum of both grids; B in units of dx
+                ContractG2P<0>(sV, sp[0], v, B);
+                ContractG2P<1>(sV, sp[1], v, B);
+                float out = 0.0f;
 #pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    const Stencil32& sg = sp[g];
-                    float m1[3];
+                for (int k = 0; k < 3; ++k) out = fmaxf(out, fabsf(sp[0].t[k] - 0.5f));
+                const bool far = !(out <= 0.5001f);
+                if (far) {
+                    MakeStencilPair(xs, sp[0], sp[1], msn, mdg);
 #pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        lw[g][k] = min(max(sg.c[k], 0), 6);
-                        const float w0 = sg.w0[k], w1 = 1.0f - w0, tt = sg.t[k];
-                        m1[k] = w1 - tt;
-                        D[k * 4] += w0 * tt * tt + w1 * (1.0f - tt) * (1.0f - tt);
-                    }
-                    D[1] += m1[0] * m1[1];
-                    D[2] += m1[0] * m1[2];
-                    D[5] += m1[1] * m1[2];
-                    const float* base = sV + g * kAWin + lw[g][0] * 64 + lw[g][1] * 8 + lw[g][2];
-                    float vg[3] = {0.f, 0.f, 0.f}, S[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int o = 0; o < 8; ++o) {
-                        const int ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
-                        const float w = NodeWeight(sg, ox, oy, oz);
-                        const int off = ox * 64 + oy * 8 + oz;
-                        const float wv[3] = {w * base[off], w * base[2 * kAWin + off], w * base[4 * kAWin + off]};
-#pragma unroll
-                        for (int r = 0; r < 3; ++r) {
-                            vg[r] += wv[r];
-                            if (ox) S[r * 3 + 0] += wv[r];
-                            if (oy) S[r * 3 + 1] += wv[r];
-                            if (oz) S[r * 3 + 2] += wv[r];
-                        }
-                    }
-#pragma unroll
-                    for (int r = 0; r < 3; ++r) {
-                        v[r] += vg[r];
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) B[r * 3 + c] += dx * (S[r * 3 + c] - vg[r] * sg.t[c]);
-                    }
+                    for (int k = 0; k < 3; ++k) v[k] = B[3 * k] = B[3 * k + 1] = B[3 * k + 2] = 0.0f;
+                    GatherG2P(0, sp[0], sHalo, a.V, v, B);
+                    GatherG2P(1, sp[1], sHalo, a.V, v, B);
                 }
                 const float dx2 = dx * dx;
-                D[0] *= dx2;
-                D[4] *= dx2;
-                D[8] *= dx2;
-                D[1] *= dx2;
-                D[2] *= dx2;
-                D[5] *= dx2;
-                D[3] = D[1];
-                D[6] = D[2];
-                D[7] = D[5];
-                float Di[9], C[9];
-                InverseSym3(D, Di);
-                MatMul3(B, Di, C);
+                // C = B D^-1; Di = D^-1 (the moments are in units of dx, B too)
+                float C[9], Di[9];
+                MomentInverse(msn, mdg, inv_dx, s6);
+                MatMulSym3(B, s6, C);
+                Unpack(s6, inv_dx, Di);
                 float xn[3];
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
@@ -389,59 +423,32 @@ __global__ __launch_bounds__(kAT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
                 for (int k = 0; k < 3; ++k) xs[k] = __fmul_rn(xn[k], inv_dx);
                 Stencil32 sn[2];
-                MakeStencilPair(xs, sn[0], sn[1]);
+                MakeStencilPair(xs, sn[0], sn[1], msn, mdg);
                 bool inwin = true;
-                float Dn[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    float m1[3];
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        const int lc = sn[g].c[k];
-                        inwin &= g == 0 ? (lc >= 1 && lc <= 6) : (lc >= 0 && lc <= 6);
-                        const float w0 = sn[g].w0[k], w1 = 1.0f - w0, tt = sn[g].t[k];
-                        m1[k] = w1 - tt;
-                        Dn[k * 4] += w0 * tt * tt + w1 * (1.0f - tt) * (1.0f - tt);
-                    }
-                    Dn[1] += m1[0] * m1[1];
-                    Dn[2] += m1[0] * m1[2];
-                    Dn[5] += m1[1] * m1[2];
-                }
+                for (int k = 0; k < 3; ++k) inwin &= static_cast<uint32_t>(sn[0].c[k] - 1) <= 5u;
                 const float h = 0.5f * dx2;
-                Dn[0] *= h;
-                Dn[4] *= h;
-                Dn[8] *= h;
-                Dn[1] *= h;
-                Dn[2] *= h;
-                Dn[5] *= h;
-                Dn[3] = Dn[1];
-                Dn[6] = Dn[2];
-                Dn[7] = Dn[5];
                 float Dh[9], DT[9], K[9];
-                InverseSym3(Dn, Dh);
+                MomentInverse(msn, mdg, 2.0f * inv_dx * inv_dx, s6);
+                Unpack(s6, 1.0f, Dh);
                 MatMul3(Dh, tau, DT);
                 const float sv_ = a.next_dt * a.mat.volume;
 #pragma unroll
                 for (int k = 0; k < 9; ++k) K[k] = C[k] * mass - sv_ * DT[k];
 
                 // ======================= backward
-                float xbn[3], Fb[9];
-#pragma unroll
-                for (int k = 0; k < 3; ++k) xbn[k] = a.xb_in[k * N + t];
-#pragma unroll
-                for (int k = 0; k < 9; ++k) Fb[k] = a.Eb_in[k * N + t];
-                float lamb = a.tb_in[t], mub = a.tb_in[N + t];
+                if (!kEarly) load_adjoints();
                 float vb[3] = {0.f, 0.f, 0.f}, Cb[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
                 if (inwin) {
                     // ---- P2G: m_i += w m;  p_i += w (m v + K xx_i), xx_i = (o - t') dx
                     float Kb[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
                     const float mv3[3] = {mass * v[0], mass * v[1], mass * v[2]};
+                    float dws[2][3];
+                    StencilSlopes(sn, dws);
 #pragma unroll
                     for (int g = 0; g < 2; ++g) {
                         const Stencil32& sg = sn[g];
-                        float dw[3];
-#pragma unroll
-                        for (int k = 0; k < 3; ++k) dw[k] = W0p(sg.t[k]);
+                        const float (&dw)[3] = dws[g];
                         const float* base = sMb + g * kAWin + sg.c[0] * 64 + sg.c[1] * 8 + sg.c[2];
 #pragma unroll
                         for (int o = 0; o < 8; ++o) {
@@ -482,12 +489,7 @@ __global__ __launch_bounds__(kAT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
                     for (int k = 0; k < 9; ++k) Dnb[k] *= sv_;
 #pragma unroll
-                    for (int g = 0; g < 2; ++g) {
-                        float dw[3];
-#pragma unroll
-                        for (int k = 0; k < 3; ++k) dw[k] = W0p(sn[g].t[k]);
-                        MomentAdjoint(sn[g], dw, Dnb, h, inv_dx, xbn);
-                    }
+                    for (int g = 0; g < 2; ++g) MomentAdjoint(sn[g], dws[g], Dnb, h, inv_dx, xbn);
                     // ---- stress: tau(F'; lambda, mu)
                     const float J = 1.0f + jm1;
                     const float trb = taub[0] + taub[4] + taub[8];
@@ -602,34 +604,56 @@ __global__ __launch_bounds__(kAT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                         Db[i * 3 + jj] = -(C[0 * 3 + i] * Bb[0 * 3 + jj] + C[1 * 3 + i] * Bb[1 * 3 + jj] +
                                            C[2 * 3 + i] * Bb[2 * 3 + jj]);
                 // ---- G2P: v = 1/2 sum w v_i;  B = sum v_i (w xx_i)^T;  D = sum w xx xx^T
+                float dwp[2][3];
+                StencilSlopes(sp, dwp);
+                // adds node o's part to x-bar; returns the node's v-bar
+                auto node = [&](const Stencil32& sg, const float (&dw)[3], int o, const float (&vi)[3], float (&vn)[3]) {
+                    const int ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
+                    const float w = NodeWeight(sg, ox, oy, oz);
+                    float gw[3];
+                    WeightGrad(sg, dw, ox, oy, oz, inv_dx, gw);
+                    const float xx[3] = {(ox - sg.t[0]) * dx, (oy - sg.t[1]) * dx, (oz - sg.t[2]) * dx};
+                    float bx[3];
+#pragma unroll
+                    for (int r = 0; r < 3; ++r) bx[r] = Bb[r * 3 + 0] * xx[0] + Bb[r * 3 + 1] * xx[1] + Bb[r * 3 + 2] * xx[2];
+                    const float ai = 0.5f * (vi[0] * vb[0] + vi[1] * vb[1] + vi[2] * vb[2]) +
+                                     vi[0] * bx[0] + vi[1] * bx[1] + vi[2] * bx[2];
+#pragma unroll
+                    for (int c = 0; c < 3; ++c)
+                        xb[c] += ai * gw[c] - w * (Bb[0 * 3 + c] * vi[0] + Bb[1 * 3 + c] * vi[1] + Bb[2 * 3 + c] * vi[2]);
+#pragma unroll
+                    for (int r = 0; r < 3; ++r) vn[r] = w * (0.5f * vb[r] + bx[r]);
+                };
 #pragma unroll
                 for (int g = 0; g < 2; ++g) {
                     const Stencil32& sg = sp[g];
-                    float dw[3];
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) dw[k] = W0p(sg.t[k]);
+                    const float (&dw)[3] = dwp[g];
                     MomentAdjoint(sg, dw, Db, dx2, inv_dx, xb);
-                    const int lbase = g * kAWin + lw[g][0] * 64 + lw[g][1] * 8 + lw[g][2];
+                    if (far) {
+#pragma unroll 1
+                        for (int o = 0; o < 8; ++o) {
+                            const int lx = min(max(sg.c[0] + ((o >> 2) & 1), 0), 7);
+                            const int ly = min(max(sg.c[1] + ((o >> 1) & 1), 0), 7), lz = min(max(sg.c[2] + (o & 1), 0), 7);
+                            const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2)];
+                            if (bi == kEmpty) continue;
+                            const size_t at = static_cast<size_t>(bi) * kVFloats + g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3);
+                            const float vi[3] = {a.V[at], a.V[at + 128], a.V[at + 256]};
+                            float vn[3];
+                            node(sg, dw, o, vi, vn);
 #pragma unroll
-                    for (int o = 0; o < 8; ++o) {
-                        const int ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
-                        const int off = lbase + ox * 64 + oy * 8 + oz;
-                        const float w = NodeWeight(sg, ox, oy, oz);
-                        float gw[3];
-                        WeightGrad(sg, dw, ox, oy, oz, inv_dx, gw);
-                        const float xx[3] = {(ox - sg.t[0]) * dx, (oy - sg.t[1]) * dx, (oz - sg.t[2]) * dx};
-                        const float vi[3] = {sV[off], sV[2 * kAWin + off], sV[4 * kAWin + off]};
-                        float bx[3];
+                            for (int r = 0; r < 3; ++r) unsafeAtomicAdd(a.Vbar + at + 128 * r, vn[r]);
+                        }
+                    } else {
+                        const int at = VEntry(g, sg.c[0], sg.c[1], sg.c[2]);
 #pragma unroll
-                        for (int r = 0; r < 3; ++r) bx[r] = Bb[r * 3 + 0] * xx[0] + Bb[r * 3 + 1] * xx[1] + Bb[r * 3 + 2] * xx[2];
-                        const float ai = 0.5f * (vi[0] * vb[0] + vi[1] * vb[1] + vi[2] * vb[2]) +
-                                         vi[0] * bx[0] + vi[1] * bx[1] + vi[2] * bx[2];
+                        for (int o = 0; o < 8; ++o) {
+                            const int off = at + ((o >> 2) & 1) * (g ? kV1X : kV0X) + ((o >> 1) & 1) * (g ? kV1Y : kV0Y) + (o & 1);
+                            const float vi[3] = {sV[off], sV[kVWin + off], sV[2 * kVWin + off]};
+                            float vn[3];
+                            node(sg, dw, o, vi, vn);
 #pragma unroll
-                        for (int c = 0; c < 3; ++c)
-                            xb[c] += ai * gw[c] - w * (Bb[0 * 3 + c] * vi[0] + Bb[1 * 3 + c] * vi[1] + Bb[2 * 3 + c] * vi[2]);
-#pragma unroll
-                        for (int r = 0; r < 3; ++r)
-                            atomicAdd(&sVb[2 * r * kAWin + off], static_cast<double>(w * (0.5f * vb[r] + bx[r])));
+                            for (int r = 0; r < 3; ++r) atomicAdd(&sVb[r * kVWin + off], static_cast<double>(vn[r]));
+                        }
                     }
                 }
 #pragma unroll
@@ -639,18 +663,22 @@ __global__ __launch_bounds__(kAT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 a.tb_out[s] = lamb;
                 a.tb_out[N + s] = mub;
             }
+            t += a.split * kBT;
+            load();
         }
         __syncthreads();
-        for (int i = tid; i < kVChannels * 2 * kAWin; i += kAT) {
-            const double val = sVb[i];
-            if (val == 0.0) continue;
-            const int ch = i / (2 * kAWin), g = (i / kAWin) & 1, l = i & (kAWin - 1);
-            const int lx = l >> 6, ly = (l >> 3) & 7, lz = l & 7;
-            const int o = ((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2);
-            const uint32_t bi = sHalo[o];
+        for (int e = tid; e < kCoreNodes; e += kBT) {
+            int g, lx, ly, lz;
+            CoreNode(e, g, lx, ly, lz);
+            const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2)];
             if (bi == kEmpty) continue;
-            const int node = g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3);
-            unsafeAtomicAdd(a.Vbar + static_cast<size_t>(bi) * kVFloats + ch * 128 + node, static_cast<float>(val));
+            const int at = VEntry(g, lx, ly, lz);
+            float* dst = a.Vbar + static_cast<size_t>(bi) * kVFloats + g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3);
+#pragma unroll
+            for (int ch = 0; ch < kVChannels; ++ch) {
+                const double val = sVb[ch * kVWin + at];
+                if (val != 0.0) unsafeAtomicAdd(dst + ch * 128, static_cast<float>(val));
+            }
         }
         __syncthreads();
     }
@@ -1227,15 +1255,15 @@ int ckmpm_adjoint_substep(ckmpm_engine* e) {
         a.lc_zero = s.lc[1];
         a.cap = e->cap;
         // few particle blocks (small scenes): several workgroups per block so that the
-        // launch still covers the 256 CUs, but no more than the block's 256-particle
+        // launch still covers the 256 CUs, but no more than the block's kBT-particle
         // chunks (a workgroup without a chunk would only hold a CU slot)
         const uint32_t blocks = std::max<uint32_t>(e->a_hint, 1);
-        const uint32_t chunks = static_cast<uint32_t>((static_cast<uint64_t>(m.n) + static_cast<uint64_t>(blocks) * kAT - 1) /
-                                                      (static_cast<uint64_t>(blocks) * kAT));
+        const uint32_t chunks = static_cast<uint32_t>((static_cast<uint64_t>(m.n) + static_cast<uint64_t>(blocks) * kBT - 1) /
+                                                      (static_cast<uint64_t>(blocks) * kBT));
         a.split = std::min<uint32_t>({8u, std::max<uint32_t>(1, (2048 + blocks) / blocks), std::max<uint32_t>(chunks, 1)});
         const uint32_t bgrid = std::min<uint32_t>(grid * a.split, 65536u / a.split * a.split);
-        if (m.kind == kFixedCorotated) G2P2GBackwardKernel<kFixedCorotated><<<bgrid, kAT, 0, st>>>(a);
-        else G2P2GBackwardKernel<kNeoHookean><<<bgrid, kAT, 0, st>>>(a);
+        if (m.kind == kFixedCorotated) G2P2GBackwardKernel<kFixedCorotated><<<bgrid, kBT, 0, st>>>(a);
+        else G2P2GBackwardKernel<kNeoHookean><<<bgrid, kBT, 0, st>>>(a);
     }
     GridBwdArgs gb{};
     gb.dom = e->dom;

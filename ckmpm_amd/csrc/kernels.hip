@@ -857,8 +857,8 @@ __global__ __launch_bounds__(kThreads) void GridUpdateKernel(GridUpdateArgs a) {
 // node, 0..7 over the block and its +1 neighbours).
 //   P2G accumulator: the particles' new stencil bases lie in [1,6] for grid 0 and [0,6]
 //     for grid 1 (window check), so nodes [1,7]^3 and [0,7]^3.
-//   velocity: the old bases lie in the block's cells 2..5 (grid 0) and 1..5 (grid 1), so
-//     nodes [2,6]^3 and [1,6]^3: 341 of the 855 entries of the accumulator's windows.
+//   velocity (stencil.h): the old bases lie in the block's cells 2..5 (grid 0) and 1..5
+//     (grid 1), so nodes [2,6]^3 and [1,6]^3: 341 of the accumulator's 855 entries.
 // Strides (in entries) of y and x.  A chunk's lanes cycle through the block's 4^3 cells,
 // z fastest, so lanes 16 apart differ by the x stride and lanes 4 apart by the y stride.
 // The 8-byte accumulator deposits of 32 such lanes fall on 32 distinct LDS bank pairs
@@ -867,13 +867,8 @@ __global__ __launch_bounds__(kThreads) void GridUpdateKernel(GridUpdateArgs a) {
 // launch from 62M to 46M, its substep from 24.8 to 24.0 ms per 40 and the 1M jelly's from
 // 6.28 to 5.77.  Padding the 4-byte velocity windows the same way gave nothing.
 constexpr int kM0Y = 8, kM0X = 60, kM1Y = 8, kM1X = 68;
-constexpr int kV0Y = 5, kV0X = 25, kV1Y = 6, kV1X = 36;
 constexpr int kM0Win = 6 * kM0X + 6 * kM0Y + 7;
 constexpr int kMWin = kM0Win + 7 * kM1X + 7 * kM1Y + 8;  // both sub-grids, one channel
-constexpr int kV0Win = 4 * kV0X + 4 * kV0Y + 5;
-constexpr int kVWin = kV0Win + 5 * kV1X + 5 * kV1Y + 6;
-constexpr int kCoreNodes = 125 + 216;    // nodes in reach of the block's own cells 2..5
-constexpr int kCoreColumns = 2 * (25 + 36);  // their z columns, one per block and (x, y)
 // Accumulator entry of node (x, y, z) of sub-grid g, or -1 for a grid-0 node outside [1,7]^3.
 __device__ __forceinline__ int MEntry(int g, int lx, int ly, int lz) {
     if (g) return kM0Win + lx * kM1X + ly * kM1Y + lz;
@@ -991,30 +986,6 @@ __device__ __forceinline__ void DepositP2G(LdsAcc* sM, const Stencil32 (&sn)[2],
     }
 }
 
-// G2P of one sub-grid from the halo blocks in global memory, for a stencil outside the
-// velocity window: adds to v (sum of both grids) and B (in units of dx).
-__device__ __forceinline__ void GatherG2P(int g, const Stencil32& s, const uint32_t* sHalo, const float* V, float (&v)[3],
-                                          float (&B)[9]) {
-#pragma unroll 1
-    for (int o = 0; o < 8; ++o) {
-        const int ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
-        const int lx = min(max(s.c[0] + ox, 0), 7), ly = min(max(s.c[1] + oy, 0), 7), lz = min(max(s.c[2] + oz, 0), 7);
-        const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2)];
-        if (bi == kEmpty) continue;
-        const float* src = V + static_cast<size_t>(bi) * kVFloats + g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3);
-        const float w = NodeWeight(s, ox, oy, oz);
-        const float d[3] = {static_cast<float>(ox) - s.t[0], static_cast<float>(oy) - s.t[1],
-                            static_cast<float>(oz) - s.t[2]};
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-            const float wv = w * src[128 * r];
-            v[r] += wv;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) B[r * 3 + c] = fmaf(wv, d[c], B[r * 3 + c]);
-        }
-    }
-}
-
 // Particles are taken in 64-particle chunks, one wavefront per chunk (chunk c of a block
 // goes to wave c mod waves): with a few hundred particles per block, 256-particle
 // chunks would leave about a quarter of the lanes idle.  The rank of a particle among
@@ -1114,27 +1085,7 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
         const float stress_q = Uniform(2.0f * a.next_dt * a.mat.volume * inv_dx * qs);
         float tmax = 0.0f;  // largest deposit bound of this thread's particles, scaled by qs
         __syncthreads();
-        // velocity halo: a thread takes a z column of 4 nodes of a grid block (16-byte loads)
-        // and stores the nodes inside the window: z = lo..3 of the block at z offset 0, 4..6
-        // of the one above
-        for (int e = tid; e < kCoreColumns; e += THREADS) {
-            const bool g1 = e < 72;
-            const int col = (g1 ? e : e - 72) >> 1, zb = e & 1, lo = g1 ? 1 : 2;
-            const int lx = (g1 ? col / 6 : col / 5) + lo, ly = col - (lx - lo) * (g1 ? 6 : 5) + lo;
-            const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | zb];
-            const float4* src = reinterpret_cast<const float4*>(a.V + static_cast<size_t>(bi) * kVFloats + (g1 ? 64 : 0) +
-                                                                (lx & 3) * 16 + (ly & 3) * 4);
-            const int r0 = (g1 ? kV0Win + (lx - 1) * kV1X + (ly - 1) * kV1Y : (lx - 2) * kV0X + (ly - 2) * kV0Y) +
-                           (zb ? 4 - lo : 0);
-#pragma unroll
-            for (int ch = 0; ch < kVChannels; ++ch) {
-                const float4 v = bi != kEmpty ? src[32 * ch] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                float* d = sV + ch * kVWin + r0;
-                d[0] = zb ? v.x : (g1 ? v.y : v.z);
-                d[1] = zb ? v.y : (g1 ? v.z : v.w);
-                if (zb || g1) d[2] = zb ? v.z : v.w;
-            }
-        }
+        StageVelocity<THREADS>(sV, a.V, sHalo, tid);
         if (tid == 0) {
             bool miss = false;
             for (int o = 0; o < 8; ++o) miss |= sHalo[o] == kEmpty;
@@ -1201,45 +1152,8 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
                         MakeStencilPair<2, 5>(xs, sp[0], sp[1], sn, diag);
                         MomentInverse(sn, diag, inv_dx, Di);
                     }
-#pragma unroll
-                    for (int g = 0; g < 2; ++g) {
-                        const Stencil32& sg = sp[g];
-                        const int s1 = g ? kV1Y : kV0Y, s2 = g ? kV1X : kV0X, lo = g ? 1 : 2;
-                        const float* base = sV + (g ? kV0Win : 0) + (sg.c[0] - lo) * s2 + (sg.c[1] - lo) * s1 + (sg.c[2] - lo);
-                        // B = sum_i v_i (x_i - x_p)^T w_i with x_i - x_p = (o - t) dx per axis:
-                        // B_rc = dx (S_rc - vg_r t_c), S_rc = sum over the nodes with o_c = 1 of w v_r.
-                        // The weights are a tensor product, so vg and S are contracted axis by
-                        // axis (z, then y, then x): 22 instructions per channel.
-                        const float wx0 = sg.w0[0], wy0 = sg.w0[1], wz0 = sg.w0[2];
-                        const float wx1 = 1.0f - wx0, wy1 = 1.0f - wy0, wz1 = 1.0f - wz0;
-#pragma unroll
-                        for (int r = 0; r < 3; ++r) {
-                            const float* vr = base + r * kVWin;
-                            float T[4], U[4];  // per (x, y) column: sum over z, z-moment
-#pragma unroll
-                            for (int q = 0; q < 4; ++q) {
-                                const int off = (q >> 1) * s2 + (q & 1) * s1;
-                                U[q] = wz1 * vr[off + 1];
-                                T[q] = fmaf(wz0, vr[off], U[q]);
-                            }
-                            float P[2], Q[2], Z[2];  // per x row: sum over y and z, y-moment, z-moment
-#pragma unroll
-                            for (int ox = 0; ox < 2; ++ox) {
-                                Q[ox] = wy1 * T[ox * 2 + 1];
-                                P[ox] = fmaf(wy0, T[ox * 2], Q[ox]);
-                                Z[ox] = fmaf(wy0, U[ox * 2], wy1 * U[ox * 2 + 1]);
-                            }
-                            const float S0 = wx1 * P[1];
-                            const float vg = fmaf(wx0, P[0], S0);
-                            const float S[3] = {S0, fmaf(wx0, Q[0], wx1 * Q[1]), fmaf(wx0, Z[0], wx1 * Z[1])};
-                            v[r] = g ? v[r] + vg : vg;
-#pragma unroll
-                            for (int c = 0; c < 3; ++c) {
-                                const float b = fmaf(-vg, sg.t[c], S[c]);
-                                B[r * 3 + c] = g ? B[r * 3 + c] + b : b;
-                            }
-                        }
-                    }
+                    ContractG2P<0>(sV, sp[0], v, B);
+                    ContractG2P<1>(sV, sp[1], v, B);
                     // A position farther out (an imported state) takes its own stencil from the
                     // grid blocks themselves; base cells beyond 1..6 are an error.
                     float out = 0.0f;
@@ -1459,13 +1373,10 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
                     // no particle left the block's cells 2..5: only nodes [2,6]^3 of grid 0
                     // and [1,6]^3 of grid 1 hold deposits, 341 of the 1024 above
                     for (int e = tid; e < kCoreNodes; e += THREADS) {
-                        const bool g1 = e < 216;
-                        const int n = g1 ? 6 : 5, q = g1 ? e : e - 216, lo = g1 ? 1 : 2;
-                        const int lx = (g1 ? q / 36 : q / 25) + lo, qy = g1 ? q / 6 : q / 5;
-                        const int ly = qy - (lx - lo) * n + lo, lz = q - qy * n + lo;
-                        const int r = MEntry(g1 ? 1 : 0, lx, ly, lz);
+                        int g, lx, ly, lz;
+                        CoreNode(e, g, lx, ly, lz);
                         flush(((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2),
-                              (g1 ? 64 : 0) + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3), r);
+                              g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3), MEntry(g, lx, ly, lz));
                     }
                 }
             }

@@ -2,7 +2,7 @@
 // base node, fractional offset t and node-0 weight w0 = 1 - t + sin(2 pi t)/(2 pi)
 // per axis; node 1 of an axis has weight 1 - w0.
 #pragma once
-#include <hip/hip_runtime.h>
+#include "common.h"
 
 namespace ckmpm {
 
@@ -120,6 +120,118 @@ __device__ __forceinline__ float NodeWeight(const Stencil32& s, int dx, int dy, 
     const float wy = dy ? 1.0f - s.w0[1] : s.w0[1];
     const float wz = dz ? 1.0f - s.w0[2] : s.w0[2];
     return wx * wy * wz;
+}
+
+// ---------------------------------------------------------------- velocity window
+// Velocities in reach of a particle block's own cells 2..5, in LDS: nodes [2,6]^3 of grid 0
+// and [1,6]^3 of grid 1 (node coordinates relative to the block's first node, 0..7 over the
+// block and its +1 neighbours).  Strides (in entries) of y and x.
+constexpr int kV0Y = 5, kV0X = 25, kV1Y = 6, kV1X = 36;
+constexpr int kV0Win = 4 * kV0X + 4 * kV0Y + 5;
+constexpr int kVWin = kV0Win + 5 * kV1X + 5 * kV1Y + 6;
+constexpr int kCoreNodes = 125 + 216;    // nodes in reach of the block's own cells 2..5
+constexpr int kCoreColumns = 2 * (25 + 36);  // their z columns, one per block and (x, y)
+// Window entry of node (x, y, z) of sub-grid g.
+__device__ __forceinline__ int VEntry(int g, int lx, int ly, int lz) {
+    return g ? kV0Win + (lx - 1) * kV1X + (ly - 1) * kV1Y + (lz - 1) : (lx - 2) * kV0X + (ly - 2) * kV0Y + (lz - 2);
+}
+// Core node e of kCoreNodes, grid 1 first.
+__device__ __forceinline__ void CoreNode(int e, int& g, int& lx, int& ly, int& lz) {
+    const bool g1 = e < 216;
+    const int n = g1 ? 6 : 5, q = g1 ? e : e - 216, lo = g1 ? 1 : 2;
+    const int qx = g1 ? q / 36 : q / 25, qy = g1 ? q / 6 : q / 5;
+    g = g1 ? 1 : 0;
+    lx = qx + lo;
+    ly = qy - qx * n + lo;
+    lz = q - qy * n + lo;
+}
+
+// Fills the window from the 2x2x2 halo blocks: a thread takes a z column of 4 nodes of a
+// grid block (16-byte loads) and stores the nodes inside the window: z = lo..3 of the block
+// at z offset 0, 4..6 of the one above.
+template <int THREADS>
+__device__ __forceinline__ void StageVelocity(float* sV, const float* V, const uint32_t* sHalo, uint32_t tid) {
+    for (int e = tid; e < kCoreColumns; e += THREADS) {
+        const bool g1 = e < 72;
+        const int col = (g1 ? e : e - 72) >> 1, zb = e & 1, lo = g1 ? 1 : 2;
+        const int lx = (g1 ? col / 6 : col / 5) + lo, ly = col - (lx - lo) * (g1 ? 6 : 5) + lo;
+        const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | zb];
+        const float4* src = reinterpret_cast<const float4*>(V + static_cast<size_t>(bi) * kVFloats + (g1 ? 64 : 0) +
+                                                            (lx & 3) * 16 + (ly & 3) * 4);
+        const int r0 = VEntry(g1 ? 1 : 0, lx, ly, zb ? 4 : lo);
+#pragma unroll
+        for (int ch = 0; ch < kVChannels; ++ch) {
+            const float4 v = bi != kEmpty ? src[32 * ch] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            float* d = sV + ch * kVWin + r0;
+            d[0] = zb ? v.x : (g1 ? v.y : v.z);
+            d[1] = zb ? v.y : (g1 ? v.z : v.w);
+            if (zb || g1) d[2] = zb ? v.z : v.w;
+        }
+    }
+}
+
+// G2P of sub-grid g from the window: v (grid 0 sets it, grid 1 adds) and B in units of dx.
+// B = sum_i v_i (x_i - x_p)^T w_i with x_i - x_p = (o - t) dx per axis:
+// B_rc = dx (S_rc - vg_r t_c), S_rc = sum over the nodes with o_c = 1 of w v_r.  The weights
+// are a tensor product, so vg and S are contracted axis by axis (z, then y, then x): 22
+// instructions per channel.
+template <int g>
+__device__ __forceinline__ void ContractG2P(const float* sV, const Stencil32& sg, float (&v)[3], float (&B)[9]) {
+    constexpr int s1 = g ? kV1Y : kV0Y, s2 = g ? kV1X : kV0X, lo = g ? 1 : 2;
+    const float* base = sV + (g ? kV0Win : 0) + (sg.c[0] - lo) * s2 + (sg.c[1] - lo) * s1 + (sg.c[2] - lo);
+    const float wx0 = sg.w0[0], wy0 = sg.w0[1], wz0 = sg.w0[2];
+    const float wx1 = 1.0f - wx0, wy1 = 1.0f - wy0, wz1 = 1.0f - wz0;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const float* vr = base + r * kVWin;
+        float T[4], U[4];  // per (x, y) column: sum over z, z-moment
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int off = (q >> 1) * s2 + (q & 1) * s1;
+            U[q] = wz1 * vr[off + 1];
+            T[q] = fmaf(wz0, vr[off], U[q]);
+        }
+        float P[2], Q[2], Z[2];  // per x row: sum over y and z, y-moment, z-moment
+#pragma unroll
+        for (int ox = 0; ox < 2; ++ox) {
+            Q[ox] = wy1 * T[ox * 2 + 1];
+            P[ox] = fmaf(wy0, T[ox * 2], Q[ox]);
+            Z[ox] = fmaf(wy0, U[ox * 2], wy1 * U[ox * 2 + 1]);
+        }
+        const float S0 = wx1 * P[1];
+        const float vg = fmaf(wx0, P[0], S0);
+        const float S[3] = {S0, fmaf(wx0, Q[0], wx1 * Q[1]), fmaf(wx0, Z[0], wx1 * Z[1])};
+        v[r] = g ? v[r] + vg : vg;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const float b = fmaf(-vg, sg.t[c], S[c]);
+            B[r * 3 + c] = g ? B[r * 3 + c] + b : b;
+        }
+    }
+}
+
+// G2P of one sub-grid from the halo blocks in global memory, for a stencil outside the
+// velocity window: adds to v (sum of both grids) and B (in units of dx).
+__device__ __forceinline__ void GatherG2P(int g, const Stencil32& s, const uint32_t* sHalo, const float* V, float (&v)[3],
+                                          float (&B)[9]) {
+#pragma unroll 1
+    for (int o = 0; o < 8; ++o) {
+        const int ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
+        const int lx = min(max(s.c[0] + ox, 0), 7), ly = min(max(s.c[1] + oy, 0), 7), lz = min(max(s.c[2] + oz, 0), 7);
+        const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2)];
+        if (bi == kEmpty) continue;
+        const float* src = V + static_cast<size_t>(bi) * kVFloats + g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3);
+        const float w = NodeWeight(s, ox, oy, oz);
+        const float d[3] = {static_cast<float>(ox) - s.t[0], static_cast<float>(oy) - s.t[1],
+                            static_cast<float>(oz) - s.t[2]};
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const float wv = w * src[128 * r];
+            v[r] += wv;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) B[r * 3 + c] = fmaf(wv, d[c], B[r * 3 + c]);
+        }
+    }
 }
 
 }  // namespace ckmpm
