@@ -1143,8 +1143,9 @@ int ckmpm_adjoint_rewind(ckmpm_engine* e, const float* vel, uint64_t nvel, const
     const LayoutBuf& L = e->L[e->cur];
     CK_HIP(e, hipMemsetAsync(e->M[e->mprev], 0, static_cast<size_t>(e->cap) * kMFloats * sizeof(float), st));
     CK_HIP(e, hipMemcpyAsync(A->host_io, vel, sizeof(float) * 3 * nvel, hipMemcpyHostToDevice, st));
-    LaunchRasterize(e->dom, A->x0[0], A->host_io, m.n, static_cast<uint32_t>(nvel), m.mat.mass, L.table, L.lc,
-                    e->M[e->mprev], e->status, st);
+    LaunchRasterize({e->dom, L.keys, L.table, L.lc, m.off[e->sc], A->setup_order[0], A->x0[0], A->host_io,
+                     static_cast<uint32_t>(nvel), m.mat.mass, e->M[e->mprev], e->status},
+                    GridSize(e), st);
     CK_HIP(e, hipMemsetAsync(m.blkmax, 0, static_cast<size_t>(e->cap) * sizeof(float), st));
     A->tlen[0] = A->tlen[1] = 0;
     A->recording = false;

@@ -476,7 +476,7 @@ int ckmpm_initial_setup(ckmpm_engine* e) {
     for (ModelBuf& m : e->models) nmax = std::max(nmax, m.n);
     float *xyz = nullptr, *vel = nullptr, *lam = nullptr, *mu = nullptr;
     uint32_t* keys = nullptr;
-    std::vector<uint32_t*> sorted(e->models.size(), nullptr);
+    std::vector<uint32_t*> sorted(e->models.size(), nullptr), ids(e->models.size(), nullptr);
     const size_t mark = e->allocs.size();
     CK_TRY(Alloc(e, &xyz, 3 * static_cast<size_t>(nmax)));
     CK_TRY(Alloc(e, &vel, 3 * static_cast<size_t>(nmax)));
@@ -502,6 +502,8 @@ int ckmpm_initial_setup(ckmpm_engine* e) {
         if (key_bits + 6 <= 32) SetupOrder(e->dom, xyz, m.n, key_bits, keys, vals, tmp, e->bitmap, e->status, s);
         else SetupOrderWide(e->dom, xyz, m.n, key_bits, keys, vals, tmp, e->bitmap, e->status, s);
         AdjointOnSetupOrder(e, i, vals, xyz);
+        CK_TRY(Alloc(e, &ids[i], m.n));
+        CK_HIP(e, hipMemcpyAsync(ids[i], vals, sizeof(uint32_t) * m.n, hipMemcpyDeviceToDevice, s));
         if (m.pp_attr) {
             CK_HIP(e, hipMemcpyAsync(lam, m.lam0.data(), sizeof(float) * m.n, hipMemcpyHostToDevice, s));
             CK_HIP(e, hipMemcpyAsync(mu, m.mu0.data(), sizeof(float) * m.n, hipMemcpyHostToDevice, s));
@@ -517,10 +519,13 @@ int ckmpm_initial_setup(ckmpm_engine* e) {
     CK_HIP(e, hipMemsetAsync(e->ext_cnt, 0, 2 * static_cast<size_t>(e->ext_tiles) * sizeof(uint32_t), s));
     ExtendLayout(e, L, true, s);
     CK_HIP(e, hipMemsetAsync(e->M[0], 0, static_cast<size_t>(e->cap) * kMFloats * sizeof(float), s));
-    for (ModelBuf& m : e->models) {
+    for (size_t i = 0; i < e->models.size(); ++i) {
+        ModelBuf& m = e->models[i];
         CK_HIP(e, hipMemcpyAsync(xyz, m.x0.data(), 3 * sizeof(float) * m.n, hipMemcpyHostToDevice, s));
         CK_HIP(e, hipMemcpyAsync(vel, m.v0.data(), 3 * sizeof(float) * m.nvel, hipMemcpyHostToDevice, s));
-        LaunchRasterize(e->dom, xyz, vel, m.n, m.nvel, m.mat.mass, L.table, L.lc, e->M[0], e->status, s);
+        // at most n of the cap blocks hold particles
+        LaunchRasterize({e->dom, L.keys, L.table, L.lc, m.off[0], ids[i], xyz, vel, m.nvel, m.mat.mass, e->M[0], e->status},
+                        GridFor(std::min(e->cap, m.n)), s);
         CK_HIP(e, hipStreamSynchronize(s));
     }
     // previous layout = setup layout (the first grid update reads M[0] through it)

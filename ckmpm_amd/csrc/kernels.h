@@ -54,8 +54,22 @@ void LaunchExportPositions(const DomainDev& d, const uint32_t* keys, const Layou
                            const float* st, uint32_t n, float* xyz, uint32_t grid, hipStream_t s);
 // Status and block counts into pinned host memory, complete once the stream is synchronised.
 void LaunchExportStatus(const Status* st, const LayoutCounts* lc, HostStatus* out, hipStream_t s);
-void LaunchRasterize(const DomainDev& d, const float* xyz, const float* vel, uint32_t n, uint32_t nvel, float mass,
-                     const uint32_t* table, const LayoutCounts* lc, float* M, Status* st, hipStream_t s);
+// Grid mass and momentum of a model's initial velocities on the setup layout, added to M.
+struct RasterizeArgs {
+    DomainDev d;
+    const uint32_t* keys;
+    const uint32_t* table;
+    const LayoutCounts* lc;
+    const uint32_t* off;   // block ranges of the setup ordering
+    const uint32_t* ids;   // input index of each position of the setup ordering
+    const float* xyz;      // input order
+    const float* vel;      // input order, or one row (nvel == 1)
+    uint32_t nvel;
+    float mass;
+    float* M;
+    Status* st;
+};
+void LaunchRasterize(const RasterizeArgs& a, uint32_t grid, hipStream_t s);
 
 // ---------------------------------------------------------------- layout
 // Map words per emit tile: the extension map is allocated in whole tiles (zero padded),

@@ -336,41 +336,94 @@ __global__ void InitStateKernel(DomainDev d, int kind, const float* xyz, const f
 }
 
 
-// mpm_algorithm.cuh:871-947 (Rasterize): m w and m w v0 on both grids, global atomics.
-__global__ void RasterizeKernel(DomainDev d, const float* xyz, const float* vel, uint32_t n, uint32_t nvel, float mass,
-                                const uint32_t* table, const LayoutCounts* lc, float* M, Status* st) {
-    const uint32_t Nb = lc->Nb;
-    for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
-        float xs[3];
+// mpm_algorithm.cuh:871-947 (Rasterize): m w and m w v0 on both grids.  A workgroup per
+// particle block of the setup layout: its particles (input indices ids[off[j]..]) deposit
+// into FP64 accumulators in LDS over the nodes in reach of the block's cells, and each
+// touched node goes to the grid with one float atomic per channel.  A particle that was
+// clamped into the domain (flagged) deposits with global atomics.  All 64 deposits of a
+// particle as global atomics took 204 us for 104k particles, 1.72 ms for 1M and 7.2 ms on
+// average for 5M and 3M; this takes 18 us, 57 us and 0.19 ms.
+__global__ __launch_bounds__(kThreads) void RasterizeKernel(RasterizeArgs a) {
+    __shared__ double sM[kMChannels * kVWin];
+    __shared__ uint32_t sHalo[8];
+    __shared__ uint32_t sMiss;  // halo blocks that are not in the grid (bits)
+    const uint32_t A = a.lc->A, Nb = a.lc->Nb, tid = threadIdx.x;
+    for (int i = tid; i < kMChannels * kVWin; i += kThreads) sM[i] = 0.0;
+    for (uint32_t j = blockIdx.x; j < A; j += gridDim.x) {
+        const uint32_t beg = a.off[j], end = a.off[j + 1];
+        if (beg == end) continue;
+        int bb[3];
+        CoordsOf(a.d, a.keys[j], bb[0], bb[1], bb[2]);
+        if (tid == 0) sMiss = 0u;
+        __syncthreads();
+        if (tid < 8) {
+            const int bx = bb[0] + ((tid >> 2) & 1), by = bb[1] + ((tid >> 1) & 1), bz = bb[2] + (tid & 1);
+            uint32_t bi = kEmpty;
+            if (InDomain(a.d, bx, by, bz)) bi = a.table[KeyOf(a.d, bx, by, bz)];
+            if (bi != kEmpty && bi >= Nb) bi = kEmpty;
+            sHalo[tid] = bi;
+            if (bi == kEmpty) atomicOr(&sMiss, 1u << tid);
+        }
+        __syncthreads();
+        const uint32_t miss = sMiss;
+        for (uint32_t t = beg + tid; t < end; t += kThreads) {
+            const uint32_t p = a.ids[t];
+            float xs[3];
 #pragma unroll
-        for (int a = 0; a < 3; ++a) xs[a] = __fmul_rn(xyz[3 * static_cast<size_t>(p) + a], d.inv_dx);
-        const float* v = nvel == 1 ? vel : vel + 3 * static_cast<size_t>(p);
-        const float v0 = v[0], v1 = v[1], v2 = v[2];
+            for (int k = 0; k < 3; ++k) xs[k] = __fmul_rn(a.xyz[3 * static_cast<size_t>(p) + k], a.d.inv_dx);
+            const float* v = a.nvel == 1 ? a.vel : a.vel + 3 * static_cast<size_t>(p);
+            const float v0 = v[0], v1 = v[1], v2 = v[2];
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            Stencil32 s;
-            if (g == 0) MakeStencil<0>(xs, s);
-            else MakeStencil<1>(xs, s);
+            for (int g = 0; g < 2; ++g) {
+                Stencil32 s;
+                if (g == 0) MakeStencil<0>(xs, s);
+                else MakeStencil<1>(xs, s);
+                uint32_t wide = 0u;  // base cell of grid 0 outside 2..5, of grid 1 outside 1..5
+                const int lo = g ? 1 : 2;
 #pragma unroll
-            for (int o = 0; o < 8; ++o) {
-                const int ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
-                const int cx = s.c[0] + ox, cy = s.c[1] + oy, cz = s.c[2] + oz;
-                const int bx = FloorDiv4(cx), by = FloorDiv4(cy), bz = FloorDiv4(cz);
-                uint32_t bi = kEmpty;
-                if (InDomain(d, bx, by, bz)) bi = table[KeyOf(d, bx, by, bz)];
-                if (bi == kEmpty || bi >= Nb) {
-                    SetFlag(st, kFlagMissingBlock);
-                    continue;
+                for (int k = 0; k < 3; ++k) wide |= static_cast<uint32_t>(s.c[k] - 4 * bb[k] - lo) > static_cast<uint32_t>(5 - lo);
+#pragma unroll
+                for (int o = 0; o < 8; ++o) {
+                    const int cx = s.c[0] + ((o >> 2) & 1), cy = s.c[1] + ((o >> 1) & 1), cz = s.c[2] + (o & 1);
+                    const float wm = NodeWeight(s, (o >> 2) & 1, (o >> 1) & 1, o & 1) * a.mass;
+                    const float q[kMChannels] = {wm, wm * v0, wm * v1, wm * v2};
+                    if (!wide) {
+                        const int lx = cx - 4 * bb[0], ly = cy - 4 * bb[1], lz = cz - 4 * bb[2];
+                        double* dst = sM + VEntry(g, lx, ly, lz);
+#pragma unroll
+                        for (int ch = 0; ch < kMChannels; ++ch) atomicAdd(dst + ch * kVWin, static_cast<double>(q[ch]));
+                        if (miss && ((miss >> (((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2))) & 1u))
+                            SetFlag(a.st, kFlagMissingBlock);
+                    } else {
+                        const int bx = FloorDiv4(cx), by = FloorDiv4(cy), bz = FloorDiv4(cz);
+                        uint32_t bi = kEmpty;
+                        if (InDomain(a.d, bx, by, bz)) bi = a.table[KeyOf(a.d, bx, by, bz)];
+                        if (bi == kEmpty || bi >= Nb) {
+                            SetFlag(a.st, kFlagMissingBlock);
+                            continue;
+                        }
+                        float* dst = a.M + static_cast<size_t>(bi) * kMFloats + g * 64 + (cx - 4 * bx) * 16 + (cy - 4 * by) * 4 + (cz - 4 * bz);
+#pragma unroll
+                        for (int ch = 0; ch < kMChannels; ++ch) unsafeAtomicAdd(dst + ch * 128, q[ch]);
+                    }
                 }
-                const int node = g * 64 + (cx - 4 * bx) * 16 + (cy - 4 * by) * 4 + (cz - 4 * bz);
-                const float wm = NodeWeight(s, ox, oy, oz) * mass;
-                float* blk = M + static_cast<size_t>(bi) * kMFloats;
-                unsafeAtomicAdd(blk + node, wm);
-                unsafeAtomicAdd(blk + 128 + node, wm * v0);
-                unsafeAtomicAdd(blk + 256 + node, wm * v1);
-                unsafeAtomicAdd(blk + 384 + node, wm * v2);
             }
         }
+        __syncthreads();
+        for (int e = tid; e < kCoreNodes; e += kThreads) {
+            int g, lx, ly, lz;
+            CoreNode(e, g, lx, ly, lz);
+            const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2)];
+            const int at = VEntry(g, lx, ly, lz);
+            float* dst = a.M + static_cast<size_t>(bi) * kMFloats + g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3);
+#pragma unroll
+            for (int ch = 0; ch < kMChannels; ++ch) {
+                const double val = sM[ch * kVWin + at];
+                sM[ch * kVWin + at] = 0.0;
+                if (val != 0.0 && bi != kEmpty) unsafeAtomicAdd(dst + ch * 128, static_cast<float>(val));
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -1782,9 +1835,8 @@ void LaunchExportStatus(const Status* st, const LayoutCounts* lc, HostStatus* ou
     static_assert(sizeof(HostStatus) == sizeof(Status) + sizeof(LayoutCounts) && sizeof(HostStatus) <= 4 * 64, "a word per lane");
     ExportStatusKernel<<<1, 64, 0, s>>>(st, lc, out);
 }
-void LaunchRasterize(const DomainDev& d, const float* xyz, const float* vel, uint32_t n, uint32_t nvel, float mass,
-                     const uint32_t* table, const LayoutCounts* lc, float* M, Status* st, hipStream_t s) {
-    RasterizeKernel<<<Blocks(n, kThreads), kThreads, 0, s>>>(d, xyz, vel, n, nvel, mass, table, lc, M, st);
+void LaunchRasterize(const RasterizeArgs& a, uint32_t grid, hipStream_t s) {
+    RasterizeKernel<<<grid, kThreads, 0, s>>>(a);
 }
 void LaunchTableInsertA(const uint32_t* keys, LayoutCounts* lc, uint32_t cap, uint32_t* table, hipStream_t s) {
     TableInsertAKernel<<<Blocks(cap, kThreads, 1024), kThreads, 0, s>>>(keys, lc, cap, table);
