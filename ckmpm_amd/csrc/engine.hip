@@ -173,7 +173,8 @@ void PhaseParticles(ckmpm_engine* e, double dt, double next_dt, FusedRec* rec = 
     // Plain calls advance the models of one workgroup size in one launch (G2P2GSet): the
     // launches are independent (their grid deposits are commutative atomic adds), and one
     // after the other each leaves a small scene's chip half empty.  Two elastic bodies of
-    // 16k particles: 111 to 81 us per substep; fluid and sand of 73k each: 155 to 127.
+    // 16k particles: 2.23 to 1.67 ms for 20 substeps and their export; fluid and sand of
+    // 73k each: 2.48 to 2.05 ms for 16.
     // Recorded launches stay separate: a graph runs them on queues of their own, which
     // overlaps different kinds better than one launch does (the 8M fluid + sand scene: 436
     // against 461 us).  The autotuner times each model alone.

@@ -730,10 +730,43 @@ constexpr int kGridIlp = 4;
 // A scene's boundary description (the reference's ProcessGridCellVelocity hook,
 // mpm_algorithm.cuh:795-799, as data): regions in order on the node's integer cell, then
 // the walls within 8 cells of the domain faces.
-__device__ __forceinline__ void ApplyBoundary(const ckmpm_boundary_desc& bc, const DomainDev& dom, const int (&cell)[3],
-                                           float (&v)[3]) {
+// What holds for every cell of a block is decided once per block: the regions that meet it
+// (bits) and the wall normal (a wall takes whole blocks: cells below 8 and from 4 dim - 8).
+// The description is read from LDS: loaded from memory at every node, it made the grid
+// update of a scene with slip walls and one region 15.7 us against 5.9 without; so it is 10.3.
+struct BlockBoundary {
+    uint32_t regions;
+    bool wall;
+    float nrm[3];  // unit length for slip walls
+};
+__device__ __forceinline__ BlockBoundary MakeBlockBoundary(const ckmpm_boundary_desc& bc, const DomainDev& dom, const int (&b)[3]) {
+    BlockBoundary o;
+    static_assert(CKMPM_MAX_REGIONS <= 32, "a bit per region");
+    o.regions = 0u;
     for (uint32_t r = 0; r < bc.nregions && r < CKMPM_MAX_REGIONS; ++r) {
-        const ckmpm_region& g = bc.regions[r];
+        bool meets = true;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) meets &= 4 * b[k] + 3 >= bc.regions[r].lo[k] && 4 * b[k] < bc.regions[r].hi[k];
+        if (meets) o.regions |= 1u << r;
+    }
+    o.wall = false;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        o.nrm[k] = b[k] < 2 ? 1.0f : (b[k] >= dom.dim[k] - 2 ? -1.0f : 0.0f);
+        o.wall |= o.nrm[k] != 0.0f;
+    }
+    o.wall &= bc.walls != CKMPM_WALLS_NONE;
+    if (o.wall && bc.walls != CKMPM_WALLS_STICKY) {
+        const float inv = rsqrtf(o.nrm[0] * o.nrm[0] + o.nrm[1] * o.nrm[1] + o.nrm[2] * o.nrm[2]);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) o.nrm[k] *= inv;
+    }
+    return o;
+}
+__device__ __forceinline__ void ApplyBoundary(const ckmpm_boundary_desc& bc, const BlockBoundary& bb, const DomainDev& dom,
+                                              const int (&cell)[3], float (&v)[3]) {
+    for (uint32_t left = bb.regions; left; left &= left - 1u) {
+        const ckmpm_region& g = bc.regions[__builtin_ctz(left)];
         bool in = true;
 #pragma unroll
         for (int k = 0; k < 3; ++k) in &= cell[k] >= g.lo[k] && cell[k] < g.hi[k];
@@ -753,25 +786,14 @@ __device__ __forceinline__ void ApplyBoundary(const ckmpm_boundary_desc& bc, con
             v[2] = g.value[0] * q[1] - g.value[1] * q[0];
         }
     }
-    if (bc.walls == CKMPM_WALLS_NONE) return;
-    float nrm[3];
-    bool on = false;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        nrm[k] = cell[k] < 8 ? 1.0f : (cell[k] >= 4 * dom.dim[k] - 8 ? -1.0f : 0.0f);
-        on |= nrm[k] != 0.0f;
-    }
-    if (!on) return;
+    if (!bb.wall) return;
     if (bc.walls == CKMPM_WALLS_STICKY) {
         v[0] = v[1] = v[2] = 0.0f;
         return;
     }
-    const float inv = rsqrtf(nrm[0] * nrm[0] + nrm[1] * nrm[1] + nrm[2] * nrm[2]);
+    const float vn = bb.nrm[0] * v[0] + bb.nrm[1] * v[1] + bb.nrm[2] * v[2];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) nrm[k] *= inv;
-    const float vn = nrm[0] * v[0] + nrm[1] * v[1] + nrm[2] * v[2];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) v[k] -= vn * nrm[k];
+    for (int k = 0; k < 3; ++k) v[k] -= vn * bb.nrm[k];
 }
 
 // kCustom: the scene's boundary description replaces the default sticky margin (a
@@ -782,6 +804,14 @@ __device__ __forceinline__ void GridUpdateBody(const GridUpdateArgs& a, uint32_t
     const uint32_t n0 = (threadIdx.x & 31u) * 4u;  // nodes n0 .. n0 + 3 of each of its blocks
     constexpr uint32_t kPer = kThreads / 32;       // blocks per workgroup and step
     const uint32_t stride = ng * kPer;
+    __shared__ ckmpm_boundary_desc sBc;
+    if constexpr (kCustom) {
+        static_assert(sizeof(ckmpm_boundary_desc) % 4 == 0, "copied by words");
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(&a.bc->d);
+        for (uint32_t i = threadIdx.x; i < sizeof(ckmpm_boundary_desc) / 4; i += kThreads)
+            reinterpret_cast<uint32_t*>(&sBc)[i] = src[i];
+        __syncthreads();
+    }
     // clear the other parity slot for the next substep (nothing else touches it now)
     if (wg == 0) {
         if (threadIdx.x == 0) a.st->vmax2_bits[a.slot ^ 1] = 0u;
@@ -821,6 +851,8 @@ __device__ __forceinline__ void GridUpdateBody(const GridUpdateArgs& a, uint32_t
             bool oob = false;
 #pragma unroll
             for (int k = 0; k < 3; ++k) oob |= (b[k] + a.dom.off[k] < 2) || (b[k] + a.dom.off[k] + 2 >= a.dom.dim[k]);
+            BlockBoundary bb{};
+            if constexpr (kCustom) bb = MakeBlockBoundary(sBc, a.dom, b);
             const float mk[4] = {m[u].x, m[u].y, m[u].z, m[u].w};
             const float pk[3][4] = {{p[u][0].x, p[u][0].y, p[u][0].z, p[u][0].w},
                                     {p[u][1].x, p[u][1].y, p[u][1].z, p[u][1].w},
@@ -836,12 +868,12 @@ __device__ __forceinline__ void GridUpdateBody(const GridUpdateArgs& a, uint32_t
 #pragma unroll
                     for (int k = 0; k < 3; ++k) v[k] = pk[k][q] * im;
                     v[1] += a.gravity * a.dt;
-                    if (kCustom) {
+                    if constexpr (kCustom) {
                         // node (x, y, z) of either sub-grid: cell 4 b + (x, y, z), as the hook sees it
                         const int cell[3] = {4 * b[0] + static_cast<int>((n >> 4) & 3u),
                                              4 * b[1] + static_cast<int>((n >> 2) & 3u),
                                              4 * b[2] + static_cast<int>(n & 3u)};
-                        ApplyBoundary(a.bc->d, a.dom, cell, v);
+                        ApplyBoundary(sBc, bb, a.dom, cell, v);
                     } else if (oob) {
                         v[0] = v[1] = v[2] = 0.0f;
                     }
