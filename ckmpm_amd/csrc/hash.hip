@@ -160,7 +160,9 @@ __global__ void HashListKernel(HashView h, BucketLists l, const uint32_t* keys, 
 }
 
 // Round R: lane l of the 32-lane group holds entry l of the bucket's list; its rank is the
-// number of entries with a smaller (key, index).  Round 0 writes every slot of the table.
+// number of entries with a smaller (key, index).  Round 0 writes every slot of the table and
+// every fill; a bucket with more entries than its list holds counts as full, since the later
+// rounds run before the host sees kBadRebuild and ask it for free slots.
 // Bounded by latency (a list, its keys, their atomics: three dependent accesses).  The sort
 // build spent 430 us on 200,003 keys, and 440 us on 25,090 with a 22 us Find of 677k keys,
 // nearly all of it on its 80 launches; this one 64 and 77 (kernels: 40 and 45).
@@ -174,7 +176,10 @@ __global__ __launch_bounds__(kHashThreads) void HashListPlaceKernel(HashView h, 
         const uint32_t c = l.cnt[static_cast<size_t>(R) * h.buckets + b];
         if (R > 0 && c == 0u) continue;
         if (c > kListEntries) {
-            if (lane == 0) atomicOr(bad, kBadRebuild);
+            if (lane == 0) {
+                atomicOr(bad, kBadRebuild);
+                if (R == 0) fill[b] = kHashBucket;
+            }
             continue;
         }
         const uint32_t f = R == 0 ? 0u : fill[b];
