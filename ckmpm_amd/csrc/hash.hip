@@ -121,10 +121,10 @@ __global__ void HashStashKernel(const uint32_t* flag, const uint32_t* pos, uint3
 }
 
 // Bucket lists of the list build.  A table at its full load has 11.2 pairs per bucket on
-// average in round 0, and a bucket of more than 32 about once in 5 million; later rounds
+// average in round 0, and a bucket of more than 32 about once in 10 million; later rounds
 // list a few percent of the pairs.  Round r's lists are list[r & 1]: round 2 reuses those
-// of round 0.  All of it lies in the build's temporaries: 67 words per bucket, of at least
-// 11.2 pairs each (6 words a pair), and one word per pair.
+// of round 0.  All of it lies in the build's temporaries (TmpWords): 67 words per bucket,
+// that is 6 to 67 per pair of the table's capacity, and one word per pair.
 constexpr uint32_t kListEntries = 32;  // half a wavefront
 constexpr uint32_t kStashSort = 1024;
 constexpr uint32_t kBadRebuild = 8u;   // error bit: this key set needs SortedBuild
@@ -408,16 +408,20 @@ HashView View(const ckmpm_hash* h) {
     return v;
 }
 
-size_t TmpWords(uint32_t m) {
-    return 10ull * m + std::max(RadixTempWords(m), ScanTempWords(m)) + 64;
-}
-
 // Table geometry for at most max_keys pairs: load factor at most 0.7 (three rounds then
 // leave almost nothing for the stash).
 uint32_t BucketsFor(uint32_t max_keys) {
     return static_cast<uint32_t>((static_cast<uint64_t>(max_keys) * 10 + 7 * kHashBucket - 1) / (7 * kHashBucket));
 }
 uint32_t StashFor(uint32_t max_keys) { return 256 + max_keys / 64; }
+
+// Words of the build's temporaries: the sort build's ten arrays and its scan or radix
+// space, or the list build's counts, lists and rest.
+size_t TmpWords(uint32_t m) {
+    const size_t sorted = 10ull * m + std::max(RadixTempWords(m), ScanTempWords(m)) + 64;
+    const size_t lists = (kHashRounds + 2ull * kListEntries) * BucketsFor(m) + 1 + m;
+    return std::max(sorted, lists);
+}
 
 // Device memory of one build: the table (slots, stash, count) and its temporaries.
 struct BuildMem {
