@@ -1004,9 +1004,16 @@ __device__ __forceinline__ int WindowOfHalo(int o, int nd) {
 // once per particle and sub-grid; each node's momenta are formed by FP64 adds, the weight
 // is converted once per node, and a deposit is one FP64 fma (w p exact in FP64, rounded
 // once) and one subtract: 2 VALU instructions per deposit.
-// e >= -64 keeps every scale 2^(kq - e) and its inverse a normal FP32 number.
+// e >= -64 keeps every scale 2^(kq - e) and its inverse a normal FP32 number.  The particle
+// loop's factors hold the scale already (m, m dx and the stress's 2 dt V / dx, times it), so
+// e also keeps the largest of them below 2^108 at the largest kq: what they are multiplied by
+// (velocities, their gradients, D^-1 <= 2^7 and the stress) then has 2^19 and more left, and
+// nothing at rest meets an infinite factor.  That floor is at work only for particles of 1/64
+// and more in those units, below speeds of about 2^-61.
 using LdsAcc = long long;
 constexpr int kMinExp = -64;
+constexpr int kMaxScale = 50;       // largest kq
+constexpr int kMaxFactorExp = 108;
 constexpr double kMagic = 6755399441055744.0;  // 1.5 * 2^52
 constexpr unsigned long long kMagicBits = 0x4338000000000000ull;
 __device__ __forceinline__ void LdsAddFixed(LdsAcc* p, double d) {
@@ -1127,6 +1134,9 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
         float ref = fmaxf(32.0f * hint, 8.0f * a.mat.mass * vmax);
         if (!(ref <= 1.0e37f)) ref = 1.0e37f;  // a non-finite grid is already flagged
         if (ref > 0.0f) mexp = max(kMinExp, static_cast<int>((__float_as_uint(ref) >> 23) & 0xFFu) - 127 + 2);
+        float factor = fmaxf(a.mat.mass * fmaxf(1.0f, dx), 2.0f * a.next_dt * a.mat.volume * inv_dx);
+        if (!(factor <= 1.0e37f)) factor = 1.0e37f;
+        mexp = max(mexp, static_cast<int>(__float_as_uint(factor) >> 23) - 127 + 1 + kMaxScale - kMaxFactorExp);
     }
 
     // The accumulator and the move counts are cleared once here; the flush and the
@@ -1163,7 +1173,7 @@ __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint3
         }
         // fixed-point scales of this block (LdsAcc): weights 2^kq, momentum 2^(kq - mexp)
         const uint32_t nblk = end - beg;
-        const int kq = min(50, 62 - (nblk > 1u ? 32 - __clz(nblk - 1u) : 0));
+        const int kq = min(kMaxScale, 62 - (nblk > 1u ? 32 - __clz(nblk - 1u) : 0));
         // powers of two built from their bit patterns: integer (scalar) arithmetic, so the
         // block-uniform scales stay in scalar registers across the particle loop
         const double wscale = __longlong_as_double(static_cast<long long>(kq + 1023) << 52);  // 2^kq
