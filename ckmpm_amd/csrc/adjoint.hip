@@ -185,27 +185,10 @@ struct AdjArgs {
     uint32_t cap;
 };
 
-// Slopes d w0 / d t = -1 + cos(2 pi t) of both sub-grids, one cosine per axis: the grids'
-// offsets differ by 1/2, so their cosines by the sign.  With f = min(t0, t1) in [0, 1/2) and
-// f' = min(f, 1/2 - f) in [0, 1/4], cos(2 pi f) = +-cos(2 pi f'), where the Taylor series
-// through x^12 is within 7e-9 (the next term, x^14 / 14!, at x = pi / 2).
+// Slopes of both sub-grids' node-0 weights per axis.
 __device__ __forceinline__ void StencilSlopes(const Stencil32 (&s)[2], float (&dw)[2][3]) {
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const float f = fminf(s[0].t[a], s[1].t[a]);
-        const float g = 0.5f - f, fp = fminf(f, g);
-        const float z = 39.47841760435743f * fp * fp;  // (2 pi f')^2
-        float p = 2.087675698786810e-09f;              //  1 / 12!
-        p = fmaf(p, z, -2.755731922398589e-07f);       // -1 / 10!
-        p = fmaf(p, z, 2.480158730158730e-05f);        //  1 / 8!
-        p = fmaf(p, z, -1.388888888888889e-03f);       // -1 / 6!
-        p = fmaf(p, z, 4.166666666666666e-02f);        //  1 / 4!
-        p = fmaf(p, z, -0.5f);
-        p = fmaf(p, z, 1.0f);
-        const float c = (g < f) != (s[0].t[a] >= 0.5f) ? -p : p;  // cos(2 pi t0)
-        dw[0][a] = c - 1.0f;
-        dw[1][a] = -1.0f - c;
-    }
+    for (int a = 0; a < 3; ++a) SlopePair(s[0].t[a], s[1].t[a], dw[0][a], dw[1][a]);
 }
 
 // Gradient (w.r.t. the position, per axis) of the node-(ox,oy,oz) weight.
