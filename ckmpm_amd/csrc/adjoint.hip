@@ -37,7 +37,27 @@ namespace {
 // Neo-Hookean: 38.5, now 28.6).
 constexpr int kBT = 128;
 constexpr int kAT = 256;         // threads per workgroup of the other kernels
-constexpr int kAWin = 512;       // 8^3 nodes of one sub-grid window
+// M-bar window of the new stencils, whose bases lie in [1,6] (grid 0) and [0,6] (grid 1): nodes
+// x = 1..7 of grid 0 and 0..7 of grid 1, y and z 0..7 of both (whole 16-byte columns).
+constexpr int kAM0 = 7 * 64, kAMWin = kAM0 + 8 * 64;
+// V-bar window: all nodes that an old stencil can reach, [1,7]^3 of grid 0 and [0,7]^3 of grid
+// 1, so that positions outside the block's own cells (an imported state) add in FP64 too.
+// 39.1 KiB with the two others: four workgroups per CU, as many as the registers allow.  A
+// window of the core nodes only, with FP32 atomics to the grid for the positions outside, lost
+// 1e-3 where 100,000 of them meet; this costs about 1 us per launch (49.0 to 50.3 us for 104k
+// fixed-corotated particles).  Strides padded off shared banks (x = 68 in grid 1) gave nothing.
+constexpr int kB0Y = 7, kB0X = 49, kB1Y = 8, kB1X = 64, kB0Win = 343, kBWin = kB0Win + 512;
+__device__ __forceinline__ int BEntry(int g, int lx, int ly, int lz) {
+    return g ? kB0Win + lx * kB1X + ly * kB1Y + lz : (lx - 1) * kB0X + (ly - 1) * kB0Y + (lz - 1);
+}
+// Node e of kBWin, grid 0 first.
+__device__ __forceinline__ void BNode(int e, int& g, int& lx, int& ly, int& lz) {
+    g = e >= kB0Win ? 1 : 0;
+    const int q = g ? e - kB0Win : e, n = g ? 8 : 7, lo = g ? 0 : 1;
+    lx = q / (n * n) + lo;
+    ly = q / n % n + lo;
+    lz = q % n + lo;
+}
 
 uint32_t AGrid(uint64_t n) {
     uint64_t b = (n + kAT - 1) / kAT;
@@ -250,9 +270,10 @@ __device__ __forceinline__ void Cofactor(const float (&F)[9], float (&c)[9]) {
 template <int KIND>
 __global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(2, 2))) void G2P2GBackwardKernel(AdjArgs a) {
     __shared__ float sV[kVChannels * kVWin];
-    __shared__ __align__(16) float sMb[kMChannels * 2 * kAWin];
-    __shared__ __align__(16) double sVb[kVChannels * kVWin + 1];  // the velocity window's adjoint
+    __shared__ __align__(16) float sMb[kMChannels * kAMWin];
+    __shared__ __align__(16) double sVb[kVChannels * kBWin + 1];
     __shared__ uint32_t sHalo[8];
+    __shared__ uint32_t sFar;  // a position lies outside the block's own cells
     // the adjoints wait until the SVD is done: held across it, they spill 14 VGPRs
     constexpr bool kEarly = KIND != kFixedCorotated;
     const uint32_t A = a.lc->A, Nb = a.lc->Nb;
@@ -313,11 +334,12 @@ __global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             if (bi != kEmpty && bi >= Nb) bi = kEmpty;
             sHalo[tid] = bi;
         }
-        for (int i = 2 * tid; i < kVChannels * kVWin; i += 2 * kBT)
+        if (tid == 0) sFar = 0u;
+        for (int i = 2 * tid; i < kVChannels * kBWin; i += 2 * kBT)
             *reinterpret_cast<uint4*>(sVb + i) = make_uint4(0u, 0u, 0u, 0u);
         __syncthreads();
-        // halo: the velocity window, and M-bar over the whole 8^3 window as 16-byte loads of a
-        // z column of a grid block, all of them in flight
+        // halo: the velocity window, and M-bar's as 16-byte loads of a z column of a grid block,
+        // all of them in flight
         StageVelocity<kBT>(sV, a.V, sHalo, tid);
         {
             constexpr int kPer = 8 * kMFloats / 4 / kBT;
@@ -330,10 +352,12 @@ __global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 q[o] = bi != kEmpty ? src[tid] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             }
             // column tid = ch * 32 + g * 16 + x * 4 + y of block o
-            const int l0 = (tid >> 4) * kAWin + ((tid >> 2) & 3) * 64 + (tid & 3) * 8;
+            const int g = (tid >> 4) & 1, lx0 = (tid >> 2) & 3;
+            const int l0 = static_cast<int>(tid >> 5) * kAMWin + (g ? kAM0 : -64) + lx0 * 64 + (tid & 3) * 8;
 #pragma unroll
             for (int o = 0; o < kPer; ++o)
-                *reinterpret_cast<float4*>(sMb + l0 + ((o >> 2) & 1) * 256 + ((o >> 1) & 1) * 32 + (o & 1) * 4) = q[o];
+                if (o >= 4 || g || lx0 > 0)
+                    *reinterpret_cast<float4*>(sMb + l0 + ((o >> 2) & 1) * 256 + ((o >> 1) & 1) * 32 + (o & 1) * 4) = q[o];
         }
         __syncthreads();
         for (uint32_t c0 = beg + part * kBT; c0 < end; c0 += a.split * kBT) {
@@ -345,7 +369,8 @@ __global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 Stencil32 sp[2];
                 float s6[6], msn[3], mdg[3];  // a symmetric matrix, the moments of the stencils
                 // base cells 2..5, as the forward takes them; a position farther out (an
-                // imported state) reads and scatters the grid blocks themselves
+                // imported state) reads the grid blocks themselves; base cells beyond 1..6,
+                // which the forward flags, count as the nearest of them
                 MakeStencilPair<2, 5>(xs, sp[0], sp[1], msn, mdg);
                 float v[3], B[9];  // v: sum of both grids; B in units of dx
                 ContractG2P<0>(sV, sp[0], v, B);
@@ -355,7 +380,8 @@ __global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 for (int k = 0; k < 3; ++k) out = fmaxf(out, fabsf(sp[0].t[k] - 0.5f));
                 const bool far = !(out <= 0.5001f);
                 if (far) {
-                    MakeStencilPair(xs, sp[0], sp[1], msn, mdg);
+                    sFar = 1u;
+                    MakeStencilPair<1, 6>(xs, sp[0], sp[1], msn, mdg);
 #pragma unroll
                     for (int k = 0; k < 3; ++k) v[k] = B[3 * k] = B[3 * k + 1] = B[3 * k + 2] = 0.0f;
                     GatherG2P(0, sp[0], sHalo, a.V, v, B);
@@ -432,7 +458,7 @@ __global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     for (int g = 0; g < 2; ++g) {
                         const Stencil32& sg = sn[g];
                         const float (&dw)[3] = dws[g];
-                        const float* base = sMb + g * kAWin + sg.c[0] * 64 + sg.c[1] * 8 + sg.c[2];
+                        const float* base = sMb + (g ? kAM0 : -64) + sg.c[0] * 64 + sg.c[1] * 8 + sg.c[2];
 #pragma unroll
                         for (int o = 0; o < 8; ++o) {
                             const int ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
@@ -442,7 +468,7 @@ __global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                             WeightGrad(sg, dw, ox, oy, oz, inv_dx, gw);
                             const float xx[3] = {(ox - sg.t[0]) * dx, (oy - sg.t[1]) * dx, (oz - sg.t[2]) * dx};
                             const float mb = base[off];
-                            const float pb[3] = {base[2 * kAWin + off], base[4 * kAWin + off], base[6 * kAWin + off]};
+                            const float pb[3] = {base[kAMWin + off], base[2 * kAMWin + off], base[3 * kAMWin + off]};
                             float gi = mb * mass;
 #pragma unroll
                             for (int r = 0; r < 3; ++r) {
@@ -612,30 +638,34 @@ __global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     const Stencil32& sg = sp[g];
                     const float (&dw)[3] = dwp[g];
                     MomentAdjoint(sg, dw, Db, dx2, inv_dx, xb);
+                    double* vb0 = sVb + BEntry(g, sg.c[0], sg.c[1], sg.c[2]);
                     if (far) {
 #pragma unroll 1
                         for (int o = 0; o < 8; ++o) {
-                            const int lx = min(max(sg.c[0] + ((o >> 2) & 1), 0), 7);
-                            const int ly = min(max(sg.c[1] + ((o >> 1) & 1), 0), 7), lz = min(max(sg.c[2] + (o & 1), 0), 7);
+                            const int ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
+                            const int lx = sg.c[0] + ox, ly = sg.c[1] + oy, lz = sg.c[2] + oz;
                             const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2)];
                             if (bi == kEmpty) continue;
-                            const size_t at = static_cast<size_t>(bi) * kVFloats + g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3);
-                            const float vi[3] = {a.V[at], a.V[at + 128], a.V[at + 256]};
+                            const float* src = a.V + static_cast<size_t>(bi) * kVFloats + g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3);
+                            const float vi[3] = {src[0], src[128], src[256]};
                             float vn[3];
                             node(sg, dw, o, vi, vn);
+                            double* dst = vb0 + ox * (g ? kB1X : kB0X) + oy * (g ? kB1Y : kB0Y) + oz;
 #pragma unroll
-                            for (int r = 0; r < 3; ++r) unsafeAtomicAdd(a.Vbar + at + 128 * r, vn[r]);
+                            for (int r = 0; r < 3; ++r) atomicAdd(dst + r * kBWin, static_cast<double>(vn[r]));
                         }
                     } else {
-                        const int at = VEntry(g, sg.c[0], sg.c[1], sg.c[2]);
+                        const float* v0 = sV + VEntry(g, sg.c[0], sg.c[1], sg.c[2]);
 #pragma unroll
                         for (int o = 0; o < 8; ++o) {
-                            const int off = at + ((o >> 2) & 1) * (g ? kV1X : kV0X) + ((o >> 1) & 1) * (g ? kV1Y : kV0Y) + (o & 1);
-                            const float vi[3] = {sV[off], sV[kVWin + off], sV[2 * kVWin + off]};
+                            const int ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
+                            const float* src = v0 + ox * (g ? kV1X : kV0X) + oy * (g ? kV1Y : kV0Y) + oz;
+                            const float vi[3] = {src[0], src[kVWin], src[2 * kVWin]};
                             float vn[3];
                             node(sg, dw, o, vi, vn);
+                            double* dst = vb0 + ox * (g ? kB1X : kB0X) + oy * (g ? kB1Y : kB0Y) + oz;
 #pragma unroll
-                            for (int r = 0; r < 3; ++r) atomicAdd(&sVb[r * kVWin + off], static_cast<double>(vn[r]));
+                            for (int r = 0; r < 3; ++r) atomicAdd(dst + r * kBWin, static_cast<double>(vn[r]));
                         }
                     }
                 }
@@ -650,16 +680,18 @@ __global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             load();
         }
         __syncthreads();
-        for (int e = tid; e < kCoreNodes; e += kBT) {
+        const bool all = sFar != 0u;  // otherwise only the core nodes hold anything
+        for (int e = tid; e < (all ? kBWin : kCoreNodes); e += kBT) {
             int g, lx, ly, lz;
-            CoreNode(e, g, lx, ly, lz);
+            if (all) BNode(e, g, lx, ly, lz);
+            else CoreNode(e, g, lx, ly, lz);
             const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2)];
             if (bi == kEmpty) continue;
-            const int at = VEntry(g, lx, ly, lz);
+            const int at = BEntry(g, lx, ly, lz);
             float* dst = a.Vbar + static_cast<size_t>(bi) * kVFloats + g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3);
 #pragma unroll
             for (int ch = 0; ch < kVChannels; ++ch) {
-                const double val = sVb[ch * kVWin + at];
+                const double val = sVb[ch * kBWin + at];
                 if (val != 0.0) unsafeAtomicAdd(dst + ch * 128, static_cast<float>(val));
             }
         }
