@@ -44,8 +44,8 @@ constexpr int kAM0 = 7 * 64, kAMWin = kAM0 + 8 * 64;
 // 1, so that positions outside the block's own cells (an imported state) add in FP64 too.
 // 39.1 KiB with the two others: four workgroups per CU, as many as the registers allow.  A
 // window of the core nodes only, with FP32 atomics to the grid for the positions outside, lost
-// 1e-3 where 100,000 of them meet; this costs about 1 us per launch (49.0 to 50.3 us for 104k
-// fixed-corotated particles).  Strides padded off shared banks (x = 68 in grid 1) gave nothing.
+// 1e-3 where 100,000 of them meet; this costs about 1 us per launch (104k fixed-corotated
+// particles: 49).  Strides padded off shared banks (x = 68 in grid 1) gave nothing.
 constexpr int kB0Y = 7, kB0X = 49, kB1Y = 8, kB1X = 64, kB0Win = 343, kBWin = kB0Win + 512;
 __device__ __forceinline__ int BEntry(int g, int lx, int ly, int lz) {
     return g ? kB0Win + lx * kB1X + ly * kB1Y + lz : (lx - 1) * kB0X + (ly - 1) * kB0Y + (lz - 1);
