@@ -267,24 +267,32 @@ int CopyOnStream(ckmpm_engine* e, void* dst, const void* src, size_t bytes, hipM
     return CKMPM_OK;
 }
 
-// The device's address of the host range [p, p + bytes), where all of it lies in one pinned
-// allocation (a kernel can then store to it: one launch in place of a staging launch and a
-// copy behind it, 16 against 26 us for the positions of 8k particles, 235 against 244 for
-// 1M; a plain copy of the state, which needs no launch, is faster as a copy); null for
-// other memory.
-void* PinnedView(void* p, size_t bytes) {
+// True where p is host memory, pageable or pinned; other memory (device, managed) is the
+// runtime's to copy to.  *view: the device's address of the range [p, p + bytes) where all of
+// it lies in one pinned allocation (a kernel can then store to it: one launch in place of a
+// staging launch and a copy behind it, 16 against 26 us for the positions of 8k particles, 235
+// against 244 for 1M; a plain copy of the state, which needs no launch, is faster as a copy),
+// else null.
+bool HostMemory(void* p, size_t bytes, void** view) {
+    *view = nullptr;
     hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();  // memory that the runtime does not know is pageable
+        return true;
+    }
+    if (at.type == hipMemoryTypeUnregistered) return true;
+    if (at.type != hipMemoryTypeHost) return false;
     hipDeviceptr_t base = nullptr;
     size_t size = 0;
     int dev = -1;
-    if (hipGetDevice(&dev) == hipSuccess && hipPointerGetAttributes(&at, p) == hipSuccess &&
-        at.type == hipMemoryTypeHost && at.devicePointer && at.device == dev &&
-        hipMemGetAddressRange(&base, &size, at.devicePointer) == hipSuccess) {
-        const size_t at0 = static_cast<char*>(at.devicePointer) - static_cast<char*>(base);
-        if (at0 <= size && bytes <= size - at0) return at.devicePointer;
+    if (hipGetDevice(&dev) != hipSuccess || !at.devicePointer || at.device != dev) return true;
+    if (hipMemGetAddressRange(&base, &size, at.devicePointer) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
     }
-    (void)hipGetLastError();  // pageable memory is not an error
-    return nullptr;
+    const size_t at0 = static_cast<char*>(at.devicePointer) - static_cast<char*>(base);
+    if (at0 <= size && bytes <= size - at0) *view = at.devicePointer;
+    return true;
 }
 
 int CheckReady(ckmpm_engine* e) {
@@ -732,17 +740,23 @@ int ckmpm_get_positions(ckmpm_engine* e, int32_t model, float* xyz, uint64_t cap
     ModelBuf& m = e->models[model];
     if (capacity < m.n) return Fail(e, CKMPM_ERR_INVALID, "capacity below particle count");
     const size_t bytes = 3 * sizeof(float) * static_cast<size_t>(m.n);
-    float* direct = static_cast<float*>(PinnedView(xyz, bytes));
-    // staging buffer for the largest model, allocated on the first call and kept (a frame
-    // loop calls this once per frame)
-    if (!direct && !e->pos_stage && !e->host_stage) {
+    void* view = nullptr;
+    const bool host = HostMemory(xyz, bytes, &view);
+    // staging buffer for the largest model, allocated when first needed and kept (a frame loop
+    // calls this once per frame)
+    float* dst = static_cast<float*>(view);
+    if (!dst) {
         uint32_t nmax = 0;
         for (const ModelBuf& q : e->models) nmax = std::max(nmax, q.n);
         const size_t most = 3 * sizeof(float) * static_cast<size_t>(nmax);
-        if (most <= kHostStageBytes) CK_HIP(e, hipHostMalloc(reinterpret_cast<void**>(&e->host_stage), most, hipHostMallocDefault));
-        else CK_TRY(Alloc(e, &e->pos_stage, 3 * static_cast<size_t>(nmax)));
+        if (host && most <= kHostStageBytes) {
+            if (!e->host_stage) CK_HIP(e, hipHostMalloc(reinterpret_cast<void**>(&e->host_stage), most, hipHostMallocDefault));
+            dst = e->host_stage;
+        } else {
+            if (!e->pos_stage) CK_TRY(Alloc(e, &e->pos_stage, 3 * static_cast<size_t>(nmax)));
+            dst = e->pos_stage;
+        }
     }
-    float* dst = direct ? direct : (e->host_stage ? e->host_stage : e->pos_stage);
     const LayoutBuf& P = e->L[1 - e->cur];
     LaunchExportPositions(e->dom, P.keys, P.lc, m.off[1 - e->sc], m.st[e->sc], m.n, dst, GridFor(e->a_hint + 8), e->stream);
     if (dst == e->pos_stage) {

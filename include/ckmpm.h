@@ -182,7 +182,9 @@ int ckmpm_get_counters(ckmpm_engine* eng, ckmpm_counters* out);
 int ckmpm_clear_flags(ckmpm_engine* eng);
 
 /* RetrieveParticleBuffer + ExportParticleToModel (mpm_algorithm.cuh:1977-2020,
- * mpm_engine.cuh:385-454): global FP32 positions of one model, AoS xyz, storage order. */
+ * mpm_engine.cuh:385-454): global FP32 positions of one model, AoS xyz, storage order.
+ * xyz is host memory, pageable or pinned (pinned is stored to directly), or device memory;
+ * it is complete on return. */
 int ckmpm_get_positions(ckmpm_engine* eng, int32_t model, float* xyz, uint64_t capacity, uint64_t* n);
 
 /* --- state export / import, in the engine's storage layout.  Used by parity tests
