@@ -1350,7 +1350,7 @@ int ckmpm_get_positions_input_order(ckmpm_engine* e, int32_t model, float* xyz) 
     JoinBack(e);  // host_io: after any undo still queued
     const LayoutBuf& P = e->L[1 - e->cur];
     const uint32_t wgs = std::max<uint32_t>(8u, std::min<uint32_t>(e->a_hint + 8u, 16384u));
-    LaunchExportPositions(e->dom, P.keys, P.lc, m.off[1 - e->sc], m.st[e->sc], n, e->pos_stage, wgs, e->stream);
+    CK_HIP(e, LaunchExportPositions(e->dom, P.keys, P.lc, m.off[1 - e->sc], m.st[e->sc], n, e->pos_stage, wgs, e->stream));
     AosToInputOrderKernel<<<AGrid(n), kAT, 0, e->stream>>>(A->ids[A->idc][model], e->pos_stage, n, A->host_io);
     CK_HIP(e, hipMemcpyAsync(xyz, A->host_io, 3 * sizeof(float) * static_cast<size_t>(n), hipMemcpyDeviceToHost, e->stream));
     CK_HIP(e, hipStreamSynchronize(e->stream));

@@ -39,8 +39,7 @@ int FlagsToCode(uint32_t f) {
 }
 
 int ReadStatus(ckmpm_engine* e, Status& st, LayoutCounts& lc) {
-    LaunchExportStatus(e->status, e->L[e->cur].lc, e->host_status, e->stream);
-    CK_HIP(e, hipGetLastError());
+    CK_HIP(e, LaunchExportStatus(e->status, e->L[e->cur].lc, e->host_status, e->stream));
     CK_HIP(e, hipStreamSynchronize(e->stream));
     st = e->host_status->st;
     lc = e->host_status->lc;
@@ -758,11 +757,11 @@ int ckmpm_get_positions(ckmpm_engine* e, int32_t model, float* xyz, uint64_t cap
         }
     }
     const LayoutBuf& P = e->L[1 - e->cur];
-    LaunchExportPositions(e->dom, P.keys, P.lc, m.off[1 - e->sc], m.st[e->sc], m.n, dst, GridFor(e->a_hint + 8), e->stream);
+    CK_HIP(e, LaunchExportPositions(e->dom, P.keys, P.lc, m.off[1 - e->sc], m.st[e->sc], m.n, dst, GridFor(e->a_hint + 8),
+                                    e->stream));
     if (dst == e->pos_stage) {
         CK_TRY(CopyOnStream(e, xyz, dst, bytes, hipMemcpyDeviceToHost));
     } else {
-        CK_HIP(e, hipGetLastError());
         CK_HIP(e, hipStreamSynchronize(e->stream));
         if (dst == e->host_stage) std::memcpy(xyz, dst, bytes);
     }

@@ -50,10 +50,12 @@ void LaunchSetupOffsets(const uint32_t* sorted_keys, uint32_t n, const uint32_t*
 void LaunchInitState(const DomainDev& d, int kind, const float* xyz, const float* lam_p, const float* mu_p, int pp_attr,
                      uint32_t* order, uint32_t n, float init, float* st, hipStream_t s, int rigid_attr = 0,
                      uint64_t rigid_count = 0);
-void LaunchExportPositions(const DomainDev& d, const uint32_t* keys, const LayoutCounts* lc, const uint32_t* off,
-                           const float* st, uint32_t n, float* xyz, uint32_t grid, hipStream_t s);
+// The launches behind the host's reads return their own status: hipGetLastError would also
+// report (and take) what another call of the thread left behind.
+hipError_t LaunchExportPositions(const DomainDev& d, const uint32_t* keys, const LayoutCounts* lc, const uint32_t* off,
+                                 const float* st, uint32_t n, float* xyz, uint32_t grid, hipStream_t s);
 // Status and block counts into pinned host memory, complete once the stream is synchronised.
-void LaunchExportStatus(const Status* st, const LayoutCounts* lc, HostStatus* out, hipStream_t s);
+hipError_t LaunchExportStatus(const Status* st, const LayoutCounts* lc, HostStatus* out, hipStream_t s);
 // Grid mass and momentum of a model's initial velocities on the setup layout, added to M.
 struct RasterizeArgs {
     DomainDev d;

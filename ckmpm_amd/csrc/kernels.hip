@@ -1877,13 +1877,16 @@ void LaunchInitState(const DomainDev& d, int kind, const float* xyz, const float
     InitStateKernel<<<Blocks(n, kThreads), kThreads, 0, s>>>(d, kind, xyz, lam_p, mu_p, pp_attr, order, n, init, st,
                                                              rigid_attr, rigid_count);
 }
-void LaunchExportPositions(const DomainDev& d, const uint32_t* keys, const LayoutCounts* lc, const uint32_t* off,
-                           const float* st, uint32_t n, float* xyz, uint32_t grid, hipStream_t s) {
-    ExportPositionsKernel<<<grid, kThreads, 0, s>>>(d, keys, lc, off, st, n, xyz);
+hipError_t LaunchExportPositions(const DomainDev& d, const uint32_t* keys, const LayoutCounts* lc, const uint32_t* off,
+                                 const float* st, uint32_t n, float* xyz, uint32_t grid, hipStream_t s) {
+    DomainDev dom = d;
+    void* args[] = {&dom, &keys, &lc, &off, &st, &n, &xyz};
+    return hipLaunchKernel(reinterpret_cast<const void*>(ExportPositionsKernel), dim3(grid), dim3(kThreads), args, 0, s);
 }
-void LaunchExportStatus(const Status* st, const LayoutCounts* lc, HostStatus* out, hipStream_t s) {
+hipError_t LaunchExportStatus(const Status* st, const LayoutCounts* lc, HostStatus* out, hipStream_t s) {
     static_assert(sizeof(HostStatus) == sizeof(Status) + sizeof(LayoutCounts) && sizeof(HostStatus) <= 4 * 64, "a word per lane");
-    ExportStatusKernel<<<1, 64, 0, s>>>(st, lc, out);
+    void* args[] = {&st, &lc, &out};
+    return hipLaunchKernel(reinterpret_cast<const void*>(ExportStatusKernel), dim3(1), dim3(64), args, 0, s);
 }
 void LaunchRasterize(const RasterizeArgs& a, uint32_t grid, hipStream_t s) {
     RasterizeKernel<<<grid, kThreads, 0, s>>>(a);
