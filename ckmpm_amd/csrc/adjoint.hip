@@ -36,24 +36,32 @@ namespace {
 // element loads of whole 8^3 windows, 48 of them in a row, had taken it to 56.7 (9k
 // Neo-Hookean: 38.5, now 28.6).
 constexpr int kBT = 128;
+// Workgroups per particle block: at most 8, or 16 while each has a slot of its own (four per
+// CU).  A block of 20,000 particles on its own: 133 us at 16, 256 at 8; one of 160,000: 795
+// and 1610; 125 blocks of 2097 Neo-Hookean particles (no slots for 16 each): 69 and 65.
+constexpr uint32_t kSplit = 8, kMaxSplit = 16, kSlots = 4 * 256;
 constexpr int kAT = 256;         // threads per workgroup of the other kernels
 // M-bar window of the new stencils, whose bases lie in [1,6] (grid 0) and [0,6] (grid 1): nodes
 // x = 1..7 of grid 0 and 0..7 of grid 1, y and z 0..7 of both (whole 16-byte columns).
 constexpr int kAM0 = 7 * 64, kAMWin = kAM0 + 8 * 64;
 // V-bar window: all nodes that an old stencil can reach, [1,7]^3 of grid 0 and [0,7]^3 of grid
 // 1, so that positions outside the block's own cells (an imported state) add in FP64 too.
-// 39.1 KiB with the two others: four workgroups per CU, as many as the registers allow.  A
+// 39.9 KiB with the two others: four workgroups per CU, as many as the registers allow.  A
 // window of the core nodes only, with FP32 atomics to the grid for the positions outside, lost
 // 1e-3 where 100,000 of them meet; this costs about 1 us per launch (104k fixed-corotated
-// particles: 49).  Strides padded off shared banks (x = 68 in grid 1) gave nothing.
-constexpr int kB0Y = 7, kB0X = 49, kB1Y = 8, kB1X = 64, kB0Win = 343, kBWin = kB0Win + 512;
+// particles: 49).  The x strides keep the deposits of neighbouring cells on other LDS banks as
+// far as the 40 KiB go: dense (49 and 64) they took 1 to 2% more, 4 to 6% where thousands of
+// particles share a cell.
+constexpr int kB0Y = 7, kB0X = 50, kB1Y = 8, kB1X = 68;
+constexpr int kB0Win = 6 * kB0X + 6 * kB0Y + 7, kBWin = kB0Win + 7 * kB1X + 7 * kB1Y + 8;
 __device__ __forceinline__ int BEntry(int g, int lx, int ly, int lz) {
     return g ? kB0Win + lx * kB1X + ly * kB1Y + lz : (lx - 1) * kB0X + (ly - 1) * kB0Y + (lz - 1);
 }
-// Node e of kBWin, grid 0 first.
+// Node e of kBNodes, grid 0 first.
+constexpr int kBNodes = 7 * 7 * 7 + 8 * 8 * 8;
 __device__ __forceinline__ void BNode(int e, int& g, int& lx, int& ly, int& lz) {
-    g = e >= kB0Win ? 1 : 0;
-    const int q = g ? e - kB0Win : e, n = g ? 8 : 7, lo = g ? 0 : 1;
+    g = e >= 343 ? 1 : 0;
+    const int q = g ? e - 343 : e, n = g ? 8 : 7, lo = g ? 0 : 1;
     lx = q / (n * n) + lo;
     ly = q / n % n + lo;
     lz = q % n + lo;
@@ -634,35 +642,44 @@ __global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     for (int r = 0; r < 3; ++r) vn[r] = w * (0.5f * vb[r] + bx[r]);
                 };
 #pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    const Stencil32& sg = sp[g];
-                    const float (&dw)[3] = dwp[g];
-                    MomentAdjoint(sg, dw, Db, dx2, inv_dx, xb);
-                    double* vb0 = sVb + BEntry(g, sg.c[0], sg.c[1], sg.c[2]);
-                    if (far) {
+                for (int g = 0; g < 2; ++g) MomentAdjoint(sp[g], dwp[g], Db, dx2, inv_dx, xb);
+                if (far) {
 #pragma unroll 1
-                        for (int o = 0; o < 8; ++o) {
-                            const int ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
-                            const int lx = sg.c[0] + ox, ly = sg.c[1] + oy, lz = sg.c[2] + oz;
-                            const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2)];
-                            if (bi == kEmpty) continue;
-                            const float* src = a.V + static_cast<size_t>(bi) * kVFloats + g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3);
-                            const float vi[3] = {src[0], src[128], src[256]};
-                            float vn[3];
-                            node(sg, dw, o, vi, vn);
-                            double* dst = vb0 + ox * (g ? kB1X : kB0X) + oy * (g ? kB1Y : kB0Y) + oz;
+                    for (int go = 0; go < 16; ++go) {
+                        const int g = go >> 3, o = go & 7, ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
+                        Stencil32 sg;
+                        float dw[3];
 #pragma unroll
-                            for (int r = 0; r < 3; ++r) atomicAdd(dst + r * kBWin, static_cast<double>(vn[r]));
+                        for (int k = 0; k < 3; ++k) {
+                            sg.c[k] = g ? sp[1].c[k] : sp[0].c[k];
+                            sg.t[k] = g ? sp[1].t[k] : sp[0].t[k];
+                            sg.w0[k] = g ? sp[1].w0[k] : sp[0].w0[k];
+                            dw[k] = g ? dwp[1][k] : dwp[0][k];
                         }
-                    } else {
+                        const int lx = sg.c[0] + ox, ly = sg.c[1] + oy, lz = sg.c[2] + oz;
+                        const uint32_t bi = sHalo[((lx >> 2) << 2) | ((ly >> 2) << 1) | (lz >> 2)];
+                        if (bi == kEmpty) continue;
+                        const float* src = a.V + static_cast<size_t>(bi) * kVFloats + g * 64 + (lx & 3) * 16 + (ly & 3) * 4 + (lz & 3);
+                        const float vi[3] = {src[0], src[128], src[256]};
+                        float vn[3];
+                        node(sg, dw, o, vi, vn);
+                        double* dst = sVb + BEntry(g, lx, ly, lz);
+#pragma unroll
+                        for (int r = 0; r < 3; ++r) atomicAdd(dst + r * kBWin, static_cast<double>(vn[r]));
+                    }
+                } else {
+#pragma unroll
+                    for (int g = 0; g < 2; ++g) {
+                        const Stencil32& sg = sp[g];
                         const float* v0 = sV + VEntry(g, sg.c[0], sg.c[1], sg.c[2]);
+                        double* vb0 = sVb + BEntry(g, sg.c[0], sg.c[1], sg.c[2]);
 #pragma unroll
                         for (int o = 0; o < 8; ++o) {
                             const int ox = (o >> 2) & 1, oy = (o >> 1) & 1, oz = o & 1;
                             const float* src = v0 + ox * (g ? kV1X : kV0X) + oy * (g ? kV1Y : kV0Y) + oz;
                             const float vi[3] = {src[0], src[kVWin], src[2 * kVWin]};
                             float vn[3];
-                            node(sg, dw, o, vi, vn);
+                            node(sg, dwp[g], o, vi, vn);
                             double* dst = vb0 + ox * (g ? kB1X : kB0X) + oy * (g ? kB1Y : kB0Y) + oz;
 #pragma unroll
                             for (int r = 0; r < 3; ++r) atomicAdd(dst + r * kBWin, static_cast<double>(vn[r]));
@@ -680,8 +697,8 @@ __global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             load();
         }
         __syncthreads();
-        const bool all = sFar != 0u;  // otherwise only the core nodes hold anything
-        for (int e = tid; e < (all ? kBWin : kCoreNodes); e += kBT) {
+        const bool all = __builtin_amdgcn_readfirstlane(sFar) != 0u;  // otherwise only the core nodes hold anything
+        for (int e = tid; e < (all ? kBNodes : kCoreNodes); e += kBT) {
             int g, lx, ly, lz;
             if (all) BNode(e, g, lx, ly, lz);
             else CoreNode(e, g, lx, ly, lz);
@@ -1276,7 +1293,8 @@ int ckmpm_adjoint_substep(ckmpm_engine* e) {
         const uint32_t blocks = std::max<uint32_t>(e->a_hint, 1);
         const uint32_t chunks = static_cast<uint32_t>((static_cast<uint64_t>(m.n) + static_cast<uint64_t>(blocks) * kBT - 1) /
                                                       (static_cast<uint64_t>(blocks) * kBT));
-        a.split = std::min<uint32_t>({8u, std::max<uint32_t>(1, (2048 + blocks) / blocks), std::max<uint32_t>(chunks, 1)});
+        const uint32_t most = std::max(std::min(kSplit, 1u + 2048u / blocks), std::min(kMaxSplit, kSlots / blocks));
+        a.split = std::min(most, std::max(chunks, 1u));
         const uint32_t bgrid = std::min<uint32_t>(grid * a.split, 65536u / a.split * a.split);
         if (m.kind == kFixedCorotated) G2P2GBackwardKernel<kFixedCorotated><<<bgrid, kBT, 0, st>>>(a);
         else G2P2GBackwardKernel<kNeoHookean><<<bgrid, kBT, 0, st>>>(a);
