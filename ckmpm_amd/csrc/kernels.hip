@@ -941,9 +941,9 @@ __global__ __launch_bounds__(kThreads) void GridUpdateKernel(GridUpdateArgs a) {
 
 // ============================================================== G2P2G
 // Fused G2P / constitutive update / P2G per particle block (mpm_algorithm.cuh:1365-1845):
-// one workgroup per particle block; the 2x2x2-block velocity halo and the P2G
-// accumulator live in LDS as 8^3 node windows of both sub-grids; each non-zero LDS
-// node is flushed once with a global float atomic.  The kernel also emits each
+// one workgroup per particle block; the velocities of the 2x2x2-block halo that the block's
+// own cells reach and the P2G accumulator live in LDS as node windows of both sub-grids; each
+// non-zero LDS node is flushed once with a global float atomic.  The kernel also emits each
 // particle's block move (direction) and its deterministic rank among the block's
 // particles with the same move, for the counting-sort rebin.
 // LDS windows of a particle block (node coordinates relative to the block's first
@@ -955,7 +955,7 @@ __global__ __launch_bounds__(kThreads) void GridUpdateKernel(GridUpdateArgs a) {
 // Strides (in entries) of y and x.  A chunk's lanes cycle through the block's 4^3 cells,
 // z fastest, so lanes 16 apart differ by the x stride and lanes 4 apart by the y stride.
 // The 8-byte accumulator deposits of 32 such lanes fall on 32 distinct LDS bank pairs
-// when x = 4 and y = 8 modulo 32; with the dense strides (7, 49 and 8, 64) two to four of
+// when x = +-4 and y = 8 modulo 32; with the dense strides (7, 49 and 8, 64) two to four of
 // them share a pair.  Padding took the bank-conflict cycles of the 5M-particle fluid
 // launch from 62M to 46M, its substep from 24.8 to 24.0 ms per 40 and the 1M jelly's from
 // 6.28 to 5.77.  Padding the 4-byte velocity windows the same way gave nothing.
@@ -999,9 +999,9 @@ __device__ __forceinline__ int WindowOfHalo(int o, int nd) {
 // so the grid's max speed that sets the CFL dt, wrong by a large factor.
 // Conversion: for an integer-valued |x| < 2^51 the FP64 sum x + 1.5 2^52 has a fixed
 // exponent and holds x in its mantissa, so x is that sum's bit pattern minus the constant
-// B = 0x4338 << 48 (whose low word is zero: one 32-bit subtract).  The momentum terms are
-// scaled by 2^s in FP32 once per particle (a power of two: exact) and converted to FP64
-// once per particle and sub-grid; each node's momenta are formed by FP64 adds, the weight
+// B = 0x4338 << 48 (whose low word is zero: one 32-bit subtract).  The momentum terms have
+// 2^s from their uniform FP32 factors (a power of two: exact) and are converted to FP64 once
+// per particle and sub-grid; each node's momenta are formed by FP64 adds, the weight
 // is converted once per node, and a deposit is one FP64 fma (w p exact in FP64, rounded
 // once) and one subtract: 2 VALU instructions per deposit.
 // e >= -64 keeps every scale 2^(kq - e) and its inverse a normal FP32 number.  The particle
@@ -1110,8 +1110,9 @@ struct G2P2GShared {
     uint32_t global;    // particles of the block deposited with global atomics
 };
 
-// 4 waves per SIMD: LDS (37.2 KiB per workgroup) allows 4 workgroups per CU; this caps
+// 4 waves per SIMD: LDS (36.3 KiB per workgroup) allows 4 workgroups per CU; this caps
 // the VGPRs at 128
+static_assert(sizeof(G2P2GShared) <= 40 * 1024, "four workgroups per CU");
 template <int KIND, int THREADS>
 __device__ __forceinline__ void G2P2GBody(const G2P2GArgs& a, uint32_t wg, uint32_t ng, G2P2GShared& sh) {
     constexpr uint32_t kWaves = THREADS / 64;

@@ -44,24 +44,6 @@ __device__ __forceinline__ float Det3(const float (&a)[9]) {
     return a[0] * (a[4] * a[8] - a[5] * a[7]) - a[1] * (a[3] * a[8] - a[5] * a[6]) + a[2] * (a[3] * a[7] - a[4] * a[6]);
 }
 
-// Inverse of a symmetric 3x3 matrix (adjugate / determinant), data_type.cuh:369-387.
-__device__ __forceinline__ void InverseSym3(const float (&a)[9], float (&r)[9]) {
-    const float c00 = a[4] * a[8] - a[5] * a[7];
-    const float c01 = a[2] * a[7] - a[1] * a[8];
-    const float c02 = a[1] * a[5] - a[2] * a[4];
-    const float c11 = a[0] * a[8] - a[2] * a[6];
-    const float c12 = a[2] * a[3] - a[0] * a[5];
-    const float c22 = a[0] * a[4] - a[1] * a[3];
-    // v_rcp_f32 (1 ulp) instead of an IEEE division sequence
-    const float id = __builtin_amdgcn_rcpf(a[0] * c00 + a[1] * (a[5] * a[6] - a[3] * a[8]) + a[2] * (a[3] * a[7] - a[4] * a[6]));
-    r[0] = id * c00;
-    r[1] = r[3] = id * c01;
-    r[2] = r[6] = id * c02;
-    r[4] = id * c11;
-    r[5] = r[7] = id * c12;
-    r[8] = id * c22;
-}
-
 // The solid state holds E = F - I (the reference stores F): an FP32 F near the identity
 // keeps only ~6e-8 absolute resolution, a large relative error of small strains; E keeps
 // full relative precision and the stresses below are evaluated from it without forming

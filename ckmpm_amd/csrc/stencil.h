@@ -124,8 +124,8 @@ __host__ __device__ __forceinline__ void SlopePair(float t0, float t1, float& d0
 }
 
 // scale * D^-1 (xx, xy, xz, yy, yz, zz), D the moment matrix of both grids in units of
-// dx^2: diag on the diagonal, 2 sn_a sn_b off it (adjugate / determinant; the reciprocal
-// is v_rcp_f32, 1 ulp).
+// dx^2: diag on the diagonal, 2 sn_a sn_b off it (adjugate / determinant, data_type.cuh:369-387;
+// the reciprocal is v_rcp_f32, 1 ulp).
 __device__ __forceinline__ void MomentInverse(const float (&sn)[3], const float (&diag)[3], float scale, float (&r)[6]) {
     const float h = 2.0f * sn[0];
     const float xy = h * sn[1], xz = h * sn[2], yz = 2.0f * sn[1] * sn[2];
