@@ -30,11 +30,11 @@ namespace {
 
 // Threads per workgroup of the particle backward.  The registers allow 8 wavefronts per CU:
 // as four workgroups of two, with a block's particles split over several, all of a small
-// scene's chunks run at once (104k fixed-corotated particles in 320 blocks: 47.8 us per
-// launch, 50.1 as two workgroups of four).  What bounds it there is the chain of memory
-// latencies (about 60% of a wavefront's cycles) and 3800 vector instructions per chunk;
+// scene's chunks run at once (104k fixed-corotated particles in 320 blocks: 48.7 us per
+// launch; two workgroups of four took 2.3 us more).  What bounds it there is the chain of
+// memory latencies (about 60% of a wavefront's cycles) and 3900 vector instructions per chunk;
 // element loads of whole 8^3 windows, 48 of them in a row, had taken it to 56.7 (9k
-// Neo-Hookean: 38.5, now 28.6).
+// Neo-Hookean: 38.5, now 30.1).
 constexpr int kBT = 128;
 // Workgroups per particle block: at most 8, or 16 while each has a slot of its own (four per
 // CU).  A block of 20,000 particles on its own: 133 us at 16, 256 at 8; one of 160,000: 795

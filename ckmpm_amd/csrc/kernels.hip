@@ -1007,7 +1007,7 @@ __device__ __forceinline__ int WindowOfHalo(int o, int nd) {
 // e >= -64 keeps every scale 2^(kq - e) and its inverse a normal FP32 number.  The particle
 // loop's factors hold the scale already (m, m dx and the stress's 2 dt V / dx, times it), so
 // e also keeps the largest of them below 2^108 at the largest kq: what they are multiplied by
-// (velocities, their gradients, D^-1 <= 2^7 and the stress) then has 2^19 and more left, and
+// (velocities, their gradients, 1 / det D <= 2^7 and the stress) has 2^19 and more left, and
 // nothing at rest meets an infinite factor.  That floor is at work only for particles of 1/64
 // and more in those units, below speeds of about 2^-61.
 using LdsAcc = long long;
